@@ -302,9 +302,11 @@ int mfx_sdpa_bwd(const mfx_sdpa_bwd_args* args, void* stream);
  * matrix-core kernels run on. */
 size_t mfx_sdpa_bwd_workspace_size(const mfx_sdpa_bwd_args* args);
 
-/* Which backward kernels mfx_sdpa_bwd would launch ("mfma_bf16_d128",
- * "mfma_bf16_d96" (through the padded copies), "generic", ...), or NULL if
- * the arguments are invalid. */
+/* Which backward kernels mfx_sdpa_bwd would launch: "mfma_bf16_d128",
+ * "mfma_bf16_d96" (through the padded copies), ... for the 16-bit
+ * matrix-core kernels; "generic" for every other call, which are the per-row
+ * kernels and, for f32 at head sizes 32, 64, 96 and 128 with 16-byte aligned
+ * rows, the fp32 matrix-core kernels.  NULL if the arguments are invalid. */
 const char* mfx_sdpa_bwd_kernel_name(const mfx_sdpa_bwd_args* args);
 
 /* ==========================================================================

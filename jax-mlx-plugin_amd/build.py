@@ -67,11 +67,12 @@ def _run(cmd: list[str]) -> None:
         print("\n".join(lines), file=sys.stderr)
 
 
-# Per-file code-generation options.  sdpa_flash_f32.hip: MFMA accumulators in
-# VGPRs rather than AGPRs (its kernels read every accumulator back into VALU
+# Per-file code-generation options.  The fp32 attention files: MFMA accumulators
+# in VGPRs rather than AGPRs (their kernels read every accumulator back into VALU
 # work -- softmax, rescale, merge -- and the AGPR form adds a move per read).
 HIP_FILE_FLAGS = {
     "sdpa_flash_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "sdpa_bwd_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 
 

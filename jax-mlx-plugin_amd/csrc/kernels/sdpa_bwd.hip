@@ -20,7 +20,9 @@
 // size 64 / 128 run on the matrix-core kernels (sdpa_bwd_mfma.hip), and head
 // sizes 32 / 96 too, on copies of q, k, v, dO and O zero-padded to 64 / 128
 // features in the workspace (the padded features add zero to every score and
-// to delta, and their gradients, zero, are not copied out).
+// to delta, and their gradients, zero, are not copied out); f32 with head
+// size 32, 64, 96 or 128 runs on the fp32 matrix-core kernels
+// (sdpa_bwd_f32.hip).
 #include <algorithm>
 #include <cmath>
 
@@ -212,6 +214,7 @@ struct BwdPlan {
   SdpaBwdParams p{};
   SdpaParams fwd{};
   bool mfma = false;
+  bool f32 = false;  // the fp32 matrix-core kernels
   size_t o_bytes = 0, row_bytes = 0;  // workspace: O, then lse, then delta
   // Head size 32 / 96 on the matrix-core kernels: pp is p on rows padded to
   // dp features (q, k, v, dO, O and dq, dk, dv in the workspace after
@@ -326,6 +329,7 @@ int make_bwd_plan(const mfx_sdpa_bwd_args* a, BwdPlan& out) {
   f.num_splits = 1;
   f.split_len = p.Tk;
   out.mfma = bwd_mfma_supports(p);
+  out.f32 = bwd_f32_supports(p);
   // The copies move 16-byte chunks: every tensor 16-byte aligned with
   // strides of whole chunks (the recomputed O is the workspace's).
   auto chunked = [&]() {
@@ -403,6 +407,7 @@ const char* mfx_sdpa_bwd_kernel_name(const mfx_sdpa_bwd_args* args) {
     static const char* const padded[2][2] = {{"mfma_bf16_d32", "mfma_bf16_d96"}, {"mfma_f16_d32", "mfma_f16_d96"}};
     return padded[pl.p.dtype == MFX_F16][pl.p.D == 96];
   }
+  // f32 calls keep the one name on either of their routes.
   if (!pl.mfma) return "generic";
   if (pl.p.dtype == MFX_F16) return pl.p.D == 128 ? "mfma_f16_d128" : "mfma_f16_d64";
   return pl.p.D == 128 ? "mfma_bf16_d128" : "mfma_bf16_d64";
@@ -442,6 +447,7 @@ int mfx_sdpa_bwd(const mfx_sdpa_bwd_args* args, void* stream) {
   }
 
   if (pl.mfma) return launch_bwd_mfma(p, s);
+  if (pl.f32) return launch_bwd_f32(p, s);
   if (pl.dp) {
     // Zero-padded copies in, the matrix-core kernels, the gradients out.
     char* w = ws + pl.o_bytes + 2 * pl.row_bytes;

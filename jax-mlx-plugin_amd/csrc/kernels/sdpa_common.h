@@ -66,6 +66,9 @@ struct SdpaBwdParams {
 bool bwd_mfma_supports(const SdpaBwdParams& p);
 // dQ (which also computes delta from O and dO), then dK and dV.
 int launch_bwd_mfma(const SdpaBwdParams& p, hipStream_t s);
+// The same in fp32 (sdpa_bwd_f32.hip).
+bool bwd_f32_supports(const SdpaBwdParams& p);
+int launch_bwd_f32(const SdpaBwdParams& p, hipStream_t s);
 
 // Kernel families; each returns MFX_OK or an error code after launching.
 int launch_flash_bf16(const SdpaParams& p, hipStream_t s);

@@ -7,7 +7,7 @@
 // K-depth of 2 per MFMA the contraction index of both products is permuted
 // so that every LDS read is a 16-byte (K) or conflict-free 4-byte (V) access
 // and V needs no transpose.  Tiles are 32 keys, double-buffered through LDS.
-#include "sdpa_common.h"
+#include "sdpa_f32.h"
 
 // 8-byte raw buffer load, bound to the LLVM intrinsic itself: this
 // compiler's __builtin_amdgcn_raw_buffer_load_b64 lowers to a 4-byte load.
@@ -38,21 +38,6 @@ bool flash_f32_use_split(const SdpaParams& p) {
 }
 
 namespace {
-
-// Bytes from the first to the last valid element of `rows` rows of D floats
-// at `stride` floats apart (0 when no row is valid).
-template <int D>
-__device__ __forceinline__ int rows_extent(int rows, int64_t stride) {
-  return rows > 0 ? (int)(((int64_t)(rows - 1) * stride + D) * 4) : 0;
-}
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t f32_rsrc(const float* base, int bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), (short)0, bytes, 0x00020000);
-}
-
-__device__ __forceinline__ f32x4 ld4(__amdgpu_buffer_rsrc_t r, int off) {
-  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
-}
 
 template <int D, bool MASK>
 struct Cfg {

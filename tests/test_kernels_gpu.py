@@ -800,6 +800,61 @@ def test_sdpa_bwd_odd_head_size_generic(cuda, nat, oracle):
     check_grads(grads, refs, "bf16")
 
 
+@pytest.mark.parametrize("D", [32, 64, 96, 128])
+@pytest.mark.parametrize("B,hq,hkv,tq,tk,causal,mdt,layout", [
+    (1, 2, 2, 33, 31, False, None, "bhtd"),  # a row past one tile, a key short of one
+    (2, 4, 2, 65, 129, False, "f32", "bthd"),
+    (1, 2, 1, 97, 64, True, "bf16", "bhtd"),  # queries past the last key
+    (1, 2, 2, 40, 130, True, "f16", "bthd"),  # keys past the last query: zero gradients
+    (16, 32, 32, 34, 34, True, None, "bhtd"),  # four wavefronts per workgroup in both kernels
+])
+def test_sdpa_bwd_f32_matrix_cores(cuda, nat, oracle, D, B, hq, hkv, tq, tk, causal, mdt, layout):
+    """The fp32 matrix-core backward at tile edges, every mask type, GQA and
+    both workgroup sizes.  Bar as the other f32 cases'; the accumulation
+    bound (D + T) * 2^-23 * sum|terms| stays below it at these sizes."""
+    shape = (lambda h, t: (B, h, t, D)) if layout == "bhtd" else (lambda h, t: (B, t, h, D))
+    mask = None
+    if mdt:
+        m = np.random.default_rng(D).standard_normal((B, 1, tq, tk)).astype(np.float32)
+        m[:, :, :, 3] = -np.inf
+        mask = dev(cuda, m, {"f32": cuda.float32, "bf16": cuda.bfloat16, "f16": cuda.float16}[mdt])
+    if B == 16:  # one batch's heads against the oracle, the others against a call of their own
+        g = cuda.Generator(device="cuda").manual_seed(D)
+        q, k, v, go = (cuda.randn(shape(h, t), generator=g, device="cuda")
+                       for h, t in ((hq, tq), (hkv, tk), (hkv, tk), (hq, tq)))
+        whole = nat.sdpa_bwd(q, k, v, go, causal=causal)
+        part = nat.sdpa_bwd(*(t[5:6].contiguous() for t in (q, k, v, go)), causal=causal)
+        refs = oracle.sdpa_bwd(*(host(t[5:6]) for t in (q, k, v, go)), 1.0 / np.sqrt(D), causal=causal, mask=None)
+        check_grads([t[5:6] for t in whole], refs, "f32")
+        check_grads(part, refs, "f32")
+        return
+    grads, refs = bwd_case(cuda, nat, oracle, 300 + D, shape(hq, tq), shape(hkv, tk), "f32", causal=causal, mask=mask,
+                           layout=layout)
+    check_grads(grads, refs, "f32")
+
+
+def test_sdpa_bwd_f32_unaligned_rows(cuda, nat, oracle):
+    """Row strides off 16 bytes and overlapping rows stay on the per-row
+    kernels, with the same gradients."""
+    import ctypes
+
+    B, H, T, D = 1, 2, 40, 64
+    rng = np.random.default_rng(77)
+    q, k, v, g = (dev(cuda, rng.standard_normal((B, H, T, D)), cuda.float32) for _ in range(4))
+    wide = cuda.zeros(B, H, T, D + 1, device="cuda")
+    wide[..., :D] = k
+    refs = nat.sdpa_bwd(q, k, v, g)
+    for a, r in zip(nat.sdpa_bwd(q, wide[..., :D], v, g), refs):
+        assert np.abs(host(a) - host(r)).max() <= F32_SDPA_TOL * max(1.0, np.abs(host(r)).max())
+    v1 = v[:, :, :1].expand(B, H, T, D)
+    dense = nat.sdpa_bwd(q, k, v1.contiguous(), g)
+    dq, dk, dv = cuda.empty_like(q), cuda.empty_like(k), cuda.empty_like(v)
+    a = nat.sdpa_bwd_args(q, k, v1, g, dq, dk, dv)
+    nat.check(nat.load().mfx_sdpa_bwd(ctypes.byref(a), ctypes.c_void_p(cuda.cuda.current_stream().cuda_stream)))
+    for o, r in zip((dq, dk, dv), dense):
+        assert np.abs(host(o) - host(r)).max() <= F32_SDPA_TOL * max(1.0, np.abs(host(r)).max())
+
+
 def test_sdpa_bwd_known_answers(cuda, nat):
     """Tk = 1: out = v, so dv = sum over query rows of dO and dq = dk = 0.
     Identical keys: P is uniform 1/Tk, so dq = 0 and every dv_j is the sum of
