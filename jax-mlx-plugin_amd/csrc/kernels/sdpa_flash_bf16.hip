@@ -54,9 +54,94 @@ using tiles::fence;
 template <int D>
 using TileLoader = tiles::TileLoader<D, kBN, kNT / 64>;
 
+// One lane's mask values of eight consecutive keys of its query row, as raw
+// bits.  MT: mask_code of the mask's type.
+//
+// Loading whole runs is what makes this kernel fast: one element at a time
+// behind a branch on the type, each load waited for alone, a
+// [1,16,1999,1999] bf16 bias took 1045 us a call on [4,16,1999,128] GQA;
+// in runs, a tile's all in flight a tile ahead, 221 (179 with 2048 keys,
+// against 129 without a mask: what is left is the mask's own vector work
+// and its loads, 32 rows of 32 bytes each).
+template <int MT>
+struct MaskRun {
+  using Elem = std::conditional_t<MT == 1, uint32_t, uint16_t>;
+  static constexpr int NW = MT == 1 ? 8 : 4;  // dwords
+  // -inf throughout, which removes the keys.
+  static constexpr uint32_t kOff = MT == 1 ? 0xFF800000u : MT == 2 ? 0xFF80FF80u : 0xFC00FC00u;
+  uint32_t w[NW + (MT != 1)];
+
+  // Keys key .. key + 7 of the row at `row` (key stride 1, at least eight
+  // keys) as 16-byte loads on any 4-byte boundary.  A run that would pass the
+  // row's end is moved back inside it; shift() undoes that.
+  //
+  // odd: some run may start on an odd 16-bit element.  Loads off a 4-byte
+  // boundary are slow (259 against 179 us with a 1999- and a 2048-key bias),
+  // so such runs load the five dwords that hold them and align() moves them
+  // into place.  (No dword without a byte of the run is touched.)
+  __device__ __forceinline__ void load(const Elem* row, int key, int Tk, bool odd) {
+    load(row + min(key, Tk - 8), odd);
+  }
+  __device__ __forceinline__ void load(const Elem* at, bool odd) {
+    typedef uint32_t run_t __attribute__((ext_vector_type(4), aligned(4)));
+    const char* from = reinterpret_cast<const char*>(reinterpret_cast<uintptr_t>(at) & ~uintptr_t(3));
+#pragma unroll
+    for (int c = 0; c < NW / 4; ++c) {
+      const run_t v = *reinterpret_cast<const run_t*>(from + c * 16);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[c * 4 + j] = v[j];
+    }
+    if constexpr (MT != 1)
+      if (odd) w[4] = *reinterpret_cast<const uint32_t*>(from + 12 + 2 * (reinterpret_cast<uintptr_t>(at) & 2));
+  }
+  // After an odd load; par: 1 when the run began on an odd element.
+  __device__ __forceinline__ void align(uint32_t par) {
+    if constexpr (MT != 1)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[j] = __builtin_amdgcn_alignbit(w[j + 1], w[j], par * 16);
+  }
+  // At a ragged end: moves the run's first valid value back to slot 0 (the
+  // slots past Tk keep something; the caller masks them).
+  __device__ __forceinline__ void shift(int key, int Tk) {
+    const int d = key - min(key, Tk - 8);
+    if constexpr (MT == 1) {
+#pragma unroll
+      for (int by = 1; by < 8; by *= 2)
+#pragma unroll
+        for (int j = 0; j + by < 8; ++j) {
+          const uint32_t a = w[j], b = w[j + by];
+          w[j] = (d & by) ? b : a;
+        }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t a = w[j], b = w[(j + 1) & 3];
+        w[j] = (d & 1) ? a >> 16 | b << 16 : a;
+      }
+#pragma unroll
+      for (int by = 1; by < 4; by *= 2)
+#pragma unroll
+        for (int j = 0; j + by < 4; ++j) {
+          const uint32_t a = w[j], b = w[j + by];
+          w[j] = (d & 2 * by) ? b : a;
+        }
+    }
+  }
+  __device__ __forceinline__ float get(int j) const {
+    if constexpr (MT == 1) return __uint_as_float(w[j]);
+    else if constexpr (MT == 2) return __uint_as_float((j & 1) ? w[j >> 1] & 0xFFFF0000u : w[j >> 1] << 16);
+    else return (j & 1) ? f16_hi(w[j >> 1]) : f16_lo(w[j >> 1]);
+  }
+};
+
+// D: LDS row width (64, 128 or 256), DV <= D: the head size.  MT: the mask's
+// type (mask_code) read in runs; kAnyMask: any type and key stride, read
+// element by element; 0: no mask (D = 256 only).
 // D = 256: one workgroup per CU (four 32 KB tiles; O, Q and S of a wavefront
 // take ~300 registers).
-template <int D, bool CAUSAL, bool MASK, int E>
+constexpr int kAnyMask = 4;
+
+template <int D, int DV, int MT, int E>
 __global__ __launch_bounds__(kNT, D > 128 ? 1 : 2) void flash_bf16_kernel(SdpaParams p) {
   __shared__ __attribute__((aligned(16))) bf16 k0[kBN * D];
   __shared__ __attribute__((aligned(16))) bf16 v0[kBN * D];
@@ -95,35 +180,77 @@ __global__ __launch_bounds__(kNT, D > 128 ? 1 : 2) void flash_bf16_kernel(SdpaPa
   const int q0 = mblk * kBM + wave * 32;
   const int qi = q0 + l32;
 
-  int kv_end = Tk;
-  // D = 256 compiles only the causal form (the other spills at this width):
-  // key j is visible to query i when j <= i + co, co = 0 for a causal call
-  // and 2^30 (every key) otherwise.
+  // Only the causal form is compiled (the other spills at D = 256): key j is
+  // visible to query i when j <= i + co, co = 0 for a causal call and 2^30
+  // (every key) otherwise.
   const int co = !p.causal ? (1 << 30) : 0;
-  if (CAUSAL) kv_end = min(Tk, min(Tq + co, (mblk + 1) * kBM + co));
+  const int kv_end = min(Tk, min(Tq + co, (mblk + 1) * kBM + co));
   const int ntiles = (kv_end + kBN - 1) / kBN;
-  const TileLoader<D> kload(kp, ks2, Tk, D, wave, lane), vload(vp, vs2, Tk, D, wave, lane);
+  const TileLoader<D> kload(kp, ks2, Tk, DV, wave, lane), vload(vp, vs2, Tk, DV, wave, lane);
   auto issue = [&](int t, bf16* kl, bf16* vl) {
     kload.load(t, kl, wave);
     vload.load(t, vl, wave);
   };
   if (ntiles > 0) issue(0, k0, v0);
+  constexpr bool MASK = MT != 0;
+  // D <= 128: the tile's mask values, loaded a tile ahead.  (D = 256 has no
+  // registers for that and loads each run where it is used.)
+  constexpr bool RUNS = MASK && MT != kAnyMask;
+  constexpr bool AHEAD = RUNS && D <= 128;
+  constexpr bool FENCE = D > 128;
+  using Run = MaskRun<RUNS ? MT : 1>;
+  Run mk[AHEAD ? kKS : 1];
+  const int64_t moff = MASK ? b * p.ms[0] + h * p.ms[1] + (int64_t)min(qi, Tq - 1) * p.ms[2] : 0;
+  const auto* mrow = static_cast<const typename Run::Elem*>(p.mask) + moff;
+  // (16-bit masks: a row, or the run at a ragged row's end, may start off a
+  // dword; row_par: this lane's row does.)
+  const bool odd =
+      RUNS && MT != 1 &&
+      (((reinterpret_cast<uintptr_t>(p.mask) >> 1) | p.ms[0] | p.ms[1] | p.ms[2] | Tk) & 1) != 0;
+  const uint32_t row_par = (uint32_t)(reinterpret_cast<uintptr_t>(mrow) >> 1) & 1;
+  auto mask_load = [&](int kb) __attribute__((always_inline)) {
+    if (kb + kBN <= Tk) {
+      const auto* at = mrow + (kb + half * 8);
+#pragma unroll
+      for (int g = 0; g < kKS; ++g) mk[AHEAD ? g : 0].load(at + g * 16, odd);
+    } else {
+#pragma unroll
+      for (int g = 0; g < kKS; ++g) mk[AHEAD ? g : 0].load(mrow, kb + g * 16 + half * 8, Tk, odd);
+    }
+  };
+  // The loaded runs of a tile put in place: `ragged` when it passes Tk.
+  auto run_place = [&](Run& run, int key, bool ragged) __attribute__((always_inline)) {
+    if (odd) run.align(row_par ^ (ragged ? min(key, Tk - 8) & 1 : 0));
+    if (ragged) run.shift(key, Tk);
+  };
+  // Whether every lane's every value is -inf.  The first value decides for
+  // nearly every tile that is not.
+  auto mask_all_off = [&]() __attribute__((always_inline)) {
+    if (__ballot(mk[0].w[0] != Run::kOff)) return false;
+    uint32_t d = 0;
+#pragma unroll
+    for (int g = 0; g < kKS; ++g)
+#pragma unroll
+      for (int j = 0; j < Run::NW; ++j) d |= mk[AHEAD ? g : 0].w[j] ^ Run::kOff;
+    return __ballot(d != 0) == 0;
+  };
+  if constexpr (AHEAD) mask_load(0);
 
   // Rows past Tq load a valid row and are zeroed, so no load is predicated.
-  bf16x8 qf[D / 16];
+  bf16x8 qf[DV / 16];
   {
     const bf16* qrow = qp + (int64_t)min(qi, Tq - 1) * qs2 + half * 8;
 #pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk) {
+    for (int kk = 0; kk < DV / 16; ++kk) {
       u32x4 raw = *reinterpret_cast<const u32x4*>(qrow + kk * 16);
       if (qi >= Tq) raw = u32x4{0u, 0u, 0u, 0u};
       qf[kk] = __builtin_bit_cast(bf16x8, raw);
     }
   }
 
-  f32x16 o[D / 32];
+  f32x16 o[DV / 32];
 #pragma unroll
-  for (int dt = 0; dt < D / 32; ++dt)
+  for (int dt = 0; dt < DV / 32; ++dt)
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[dt][i] = 0.f;
   // Running exp2 base (log2 units, shared by lanes l and l^32) and the
@@ -131,23 +258,44 @@ __global__ __launch_bounds__(kNT, D > 128 ? 1 : 2) void flash_bf16_kernel(SdpaPa
   float b_run = -INFINITY, l_run = 0.f;
   const float sl2 = p.scale_log2;  // > 0 (checked on the host)
 
-  // Per-lane LDS offsets (bf16 elements) of the operand reads.
-  const int k_off = l32 * D;            // + mt*32*D, chunk (kk*2 + half) ^ k_sw
-  const int k_sw = tile_swz<D>(l32);
+  // Per-lane LDS byte offsets of the operand reads.  Row r of a 32-key score
+  // block is key r with bits 2 and 3 swapped, so that a lane's scores of a
+  // 16-key step belong to eight consecutive keys, half*8 + (0..7): a run of
+  // the mask's row.  The swizzle xors chunk bits below the row's, so chunk
+  // c + 2j (K) and c + 4j (V) of a row are the first one's offset xor 32j, 64j.
+  const int k_row = (l32 & ~12) | (l32 & 4) << 1 | (l32 & 8) >> 1;
+  const uint32_t k_off = k_row * D * 2 + (half ^ tile_swz<D>(k_row)) * 16;
   const int tj = lane & 15, tg = (lane >> 4) & 1;
-  const int v_row = 4 * half + (tj >> 2);  // + ks*16 + 8*r
-  const int v_sw = tile_swz<D>(v_row), v_sw8 = tile_swz<D>(v_row + 8);
-  const int v_chunk = tg * 2 + ((tj & 3) >> 1);  // + dt*4
-  const int v_sub = (tj & 1) * 4;
+  const int v_row = 8 * half + (tj >> 2);  // + ks*16 + 4*r
+  const int v_chunk = tg * 2 + ((tj & 3) >> 1);
+  const uint32_t v_off = v_row * D * 2 + (v_chunk ^ tile_swz<D>(v_row)) * 16 + (tj & 1) * 8;
+  const uint32_t v_off4 = (v_row + 4) * D * 2 + (v_chunk ^ tile_swz<D>(v_row + 4)) * 16 + (tj & 1) * 8;
 
   // One 64-key tile for this wave's 32 queries.  EDGE tiles (ragged end,
   // causal diagonal) mask per element; interior tiles do no mask work.
   auto compute = [&](const bf16* kl, const bf16* vl, int kb, auto edge_tag) {
     constexpr bool EDGE = decltype(edge_tag)::value;
-    // D = 256: the phases of a tile (S, softmax, PV) and the tiles stay
-    // apart, so no tile's fragments are live across another's.
-    if constexpr (D > 128) fence();
+    // Opaque: otherwise every chunk's offset into each of the four arrays is
+    // hoisted out of the loop into a register of its own, and D = 128 spills.
+    uint32_t ka = k_off, va = v_off, va4 = v_off4;
+    asm volatile("" : "+v"(ka), "+v"(va), "+v"(va4));
+    const char* kb8 = reinterpret_cast<const char*>(kl);
+    const char* vb8 = reinterpret_cast<const char*>(vl);
+    const bool more = kb + kBN < kv_end;
+    if constexpr (AHEAD) {
+      const bool ragged = EDGE && kb + kBN > Tk;
+      if (odd || ragged)
+#pragma unroll
+        for (int g = 0; g < kKS; ++g) run_place(mk[g], kb + g * 16 + half * 8, ragged);
+    }
+    // Nothing visible: a band or block mask's tiles outside it.
+    const bool off = AHEAD && mask_all_off();
     f32x16 s[kMT];
+    float mx = -INFINITY;
+    if (!off) {
+    // Where registers are short, the phases of a tile (S, softmax, PV) and
+    // the tiles stay apart, so no tile's fragments are live across another's.
+    if constexpr (FENCE) fence();
     // The two waves of a SIMD alternate between MFMA blocks and softmax
     // work; raising a wave's priority for its MFMA blocks lets the arbiter
     // keep the matrix core fed while the other wave's vector work fills in.
@@ -157,38 +305,78 @@ __global__ __launch_bounds__(kNT, D > 128 ? 1 : 2) void flash_bf16_kernel(SdpaPa
 #pragma unroll
       for (int i = 0; i < 16; ++i) s[mt][i] = 0.f;
 #pragma unroll
-      for (int kk = 0; kk < D / 16; ++kk) {
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(&kl[mt * 32 * D + k_off + ((kk * 2 + half) ^ k_sw) * 8]);
+      for (int kk = 0; kk < DV / 16; ++kk) {
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(kb8 + mt * 32 * D * 2 + (ka ^ kk * 32));
         s[mt] = mfma16<E>(a, qf[kk], s[mt]);
-        // D = 256: at most four operand reads run ahead of their MFMAs (all
-        // of a tile's at once do not fit the registers).
-        if constexpr (D > 128)
+        // ... and at most four operand reads run ahead of their MFMAs.
+        if constexpr (FENCE)
           if ((kk & 3) == 3) fence();
       }
     }
     __builtin_amdgcn_s_setprio(0);
-    if constexpr (D > 128) fence();
+    if constexpr (FENCE) fence();
     // MASK: scores move to the log2 domain here (scale and mask folded);
     // otherwise they stay raw and the scale is folded into the exp2 FMA.
-    float mx = -INFINITY;
+    // Score i of block mt is slot i & 7 of step mt*2 + (i >> 3).
+    //
+    // mask_log2's clamp keeps -inf; here -inf takes part as the clamp value
+    // (one instruction fewer per clause), whose exp2 is 0 all the same beside
+    // any row base above -1e37, and is put back where no key of a row has
+    // come near that yet.  (f16 masks have no value below the clamp.)
+    // EDGE: the last key of the tile the query sees, counted from the lane's
+    // first (opaque, or its 32 comparands are hoisted out of the loop).
+    int lim = min(qi + co, Tk - 1) - kb - half * 8;
+    if constexpr (EDGE) asm volatile("" : "+v"(lim));
 #pragma unroll
     for (int mt = 0; mt < kMT; ++mt)
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         float x = s[mt][i];
-        const int key = kb + mt * 32 + (i >> 2) * 8 + half * 4 + (i & 3);
-        if constexpr (MASK) {
-          x *= sl2;
-          if (qi < Tq && key < Tk)
-            x += mask_log2(load_mask(p.mask, p.mask_dtype,
-                                    b * p.ms[0] + h * p.ms[1] + qi * p.ms[2] + key * p.ms[3]));
+        const int g = mt * 2 + (i >> 3), key = kb + g * 16 + half * 8 + (i & 7);
+        if constexpr (MT == kAnyMask) {
+          x = x * sl2 + mask_log2(load_mask(p.mask, p.mask_dtype, moff + min(key, Tk - 1) * p.ms[3]));
+        } else if constexpr (MASK) {
+          Run& run = mk[AHEAD ? g : 0];
+          if constexpr (!AHEAD)
+            if ((i & 7) == 0) {
+              fence();
+              run.load(mrow, key, Tk, odd);
+              run_place(run, key, EDGE && kb + kBN > Tk);
+            }
+          float m = run.get(i & 7);
+          if constexpr (AHEAD) {
+            if constexpr (MT != 3) m = __builtin_elementwise_maximum(m, kMaskMin);
+            x = fmaf(m, kLog2e, x * sl2);
+          } else {
+            x = x * sl2 + mask_log2(m);
+          }
         }
         if constexpr (EDGE) {
-          if (key >= Tk || (CAUSAL && key > qi + co)) x = -INFINITY;
+          if (g * 16 + (i & 7) > lim) x = -INFINITY;
         }
         s[mt][i] = x;
         mx = fmaxf(mx, x);
+        if constexpr (FENCE && AHEAD)
+          if ((i & 3) == 3) fence();
       }
+    if constexpr (AHEAD && MT != 3) {
+      if (__ballot(fmaxf(mx, b_run) < -1e37f)) {
+        mx = -INFINITY;
+#pragma unroll
+        for (int mt = 0; mt < kMT; ++mt)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            if (mk[AHEAD ? mt * 2 + (i >> 3) : 0].get(i & 7) == -INFINITY) s[mt][i] = -INFINITY;
+            mx = fmaxf(mx, s[mt][i]);
+          }
+      }
+    }
+    }
+    // The next tile's mask, on its way under this tile's exps and PV.
+    if constexpr (AHEAD) {
+      if (more) mask_load(kb + kBN);
+      if (off) return;
+    }
     // Lanes l and l^32 hold the two halves of one query's keys.
     {
       const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
@@ -202,7 +390,7 @@ __global__ __launch_bounds__(kNT, D > 128 ? 1 : 2) void flash_bf16_kernel(SdpaPa
       b_run = nb;
       l_run *= alpha;
 #pragma unroll
-      for (int dt = 0; dt < D / 32; ++dt)
+      for (int dt = 0; dt < DV / 32; ++dt)
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
     }
@@ -245,30 +433,28 @@ __global__ __launch_bounds__(kNT, D > 128 ? 1 : 2) void flash_bf16_kernel(SdpaPa
       for (int j = 0; j < kKS; ++j) pb[j] = __builtin_bit_cast(bf16x8, pw[j]);
     }
     l_run += l0 + l1;
-    if constexpr (D > 128) fence();
+    if constexpr (FENCE) fence();
     __builtin_amdgcn_s_setprio(3);
 #pragma unroll
-    for (int dt = 0; dt < D / 32; ++dt)
+    for (int dt = 0; dt < DV / 32; ++dt)
 #pragma unroll
       for (int ks = 0; ks < kKS; ++ks) {
-        // k-slots 0-3: keys ks*16 + 4*half + e; slots 4-7: the same + 8.
-        const bf16* v_rows = vl + (ks * 16 + v_row) * D + v_sub;
-        const s16x4 lo =
-            __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(v_rows + ((dt * 4 + v_chunk) ^ v_sw) * 8));
-        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (lds_s16x4_t*)(v_rows + 8 * D + ((dt * 4 + v_chunk) ^ v_sw8) * 8));
+        // k-slots 0-3: keys ks*16 + 8*half + e; slots 4-7: the same + 4.
+        const char* v_rows = vb8 + ks * 16 * D * 2;
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(v_rows + (va ^ dt * 64)));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(v_rows + (va4 ^ dt * 64)));
         const bf16x8 a = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
         o[dt] = mfma16<E>(a, pb[ks], o[dt]);
-        if constexpr (D > 128)
+        if constexpr (FENCE)
           if ((ks & 1) == 1) fence();
       }
-    if constexpr (D > 128) fence();
+    if constexpr (FENCE) fence();
   };
 
-  auto step = [&](int t, const bf16* kl, const bf16* vl) {
+  auto step = [&](int t, const bf16* kl, const bf16* vl) __attribute__((always_inline)) {
     const int kb = t * kBN;
-    if (q0 >= Tq || (CAUSAL && kb > q0 + 31 + co)) return;  // nothing of this tile is visible
-    const bool edge = (kb + kBN > Tk) || (CAUSAL && kb + kBN - 1 > q0 + co);
+    if (q0 >= Tq || kb > q0 + 31 + co) return;  // nothing of this tile is visible
+    const bool edge = (kb + kBN > Tk) || (kb + kBN - 1 > q0 + co);
     if (edge)
       compute(kl, vl, kb, std::true_type{});
     else
@@ -300,7 +486,7 @@ __global__ __launch_bounds__(kNT, D > 128 ? 1 : 2) void flash_bf16_kernel(SdpaPa
   const float lt = l_run + __shfl_xor(l_run, 32, 64);
   const float inv = 1.0f / lt;
   if (p.lse && half == 0 && qi < Tq) p.lse[(int64_t)bh * Tq + qi] = b_run + __log2f(lt);
-  if constexpr (D <= 128) {
+  if constexpr (D <= 128 && DV == D) {
     // Every iteration ended at a barrier after its reads and with no load in
     // flight: the tile arrays take the output rows on their way out (k0
     // holds wavefronts 0 and 1, v0 wavefronts 2 and 3), stored as whole
@@ -314,7 +500,7 @@ __global__ __launch_bounds__(kNT, D > 128 ? 1 : 2) void flash_bf16_kernel(SdpaPa
   } else if (qi < Tq) {
     bf16* orow = op + qi * os2;
 #pragma unroll
-    for (int dt = 0; dt < D / 32; ++dt)
+    for (int dt = 0; dt < DV / 32; ++dt)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         u16x4 w;
@@ -325,25 +511,35 @@ __global__ __launch_bounds__(kNT, D > 128 ? 1 : 2) void flash_bf16_kernel(SdpaPa
   }
 }
 
-template <int D, bool CAUSAL, bool MASK, int E>
+template <int D, int DV, int MT, int E>
 int launch_t(const SdpaParams& p, hipStream_t s) {
   const int nmb = (p.Tq + kBM - 1) / kBM;
   const int64_t blocks = (int64_t)nmb * p.B * p.Hq;
-  hipLaunchKernelGGL((flash_bf16_kernel<D, CAUSAL, MASK, E>), dim3((unsigned)blocks), dim3(kNT), 0, s, p);
+  hipLaunchKernelGGL((flash_bf16_kernel<D, DV, MT, E>), dim3((unsigned)blocks), dim3(kNT), 0, s, p);
   return launch_status("flash_bf16_kernel");
 }
 
-template <int D, int E>
-int launch_d(const SdpaParams& p, hipStream_t s) {
-  return launch_t<D, true, true, E>(p, s);
+template <int D, int DV, int E>
+int launch_m(const SdpaParams& p, hipStream_t s) {
+  if (p.ms[3] != 1 || p.Tk < 8) return launch_t<D, DV, kAnyMask, E>(p, s);
+  switch (mask_code(p.mask_dtype)) {
+    case 1: return launch_t<D, DV, 1, E>(p, s);
+    case 2: return launch_t<D, DV, 2, E>(p, s);
+    default: return launch_t<D, DV, 3, E>(p, s);
+  }
 }
 
-// Head size 256, every mask form (the pipelined kernel stops at 128): the
-// causal instantiations serve non-causal calls too (through the kernel's
-// causal offset).
+// Head size 256 comes here in every mask form (the pipelined kernel stops at
+// 128).
 template <int E>
-int launch_256(const SdpaParams& p, hipStream_t s) {
-  return p.mask ? launch_t<256, true, true, E>(p, s) : launch_t<256, true, false, E>(p, s);
+int launch_d(const SdpaParams& p, hipStream_t s) {
+  switch (p.D) {
+    case 32: return launch_m<64, 32, E>(p, s);
+    case 64: return launch_m<64, 64, E>(p, s);
+    case 96: return launch_m<128, 96, E>(p, s);
+    case 128: return launch_m<128, 128, E>(p, s);
+    default: return p.mask ? launch_m<256, 256, E>(p, s) : launch_t<256, 256, 0, E>(p, s);
+  }
 }
 
 bool aligned16(const void* ptr) { return ((uintptr_t)ptr & 15) == 0; }
@@ -361,9 +557,6 @@ bool flash_bf16_supports(const SdpaParams& p) {
   if (p.ks[2] < p.D || p.vs[2] < p.Dv) return false;
   if ((int64_t)p.Tk * p.ks[2] * 2 >= (1LL << 31) || (int64_t)p.Tk * p.vs[2] * 2 >= (1LL << 31)) return false;
   if (p.D != p.Dv || (p.D != 32 && p.D != 64 && p.D != 96 && p.D != 128 && p.D != 256)) return false;
-  // Masks that vary along query rows run on this file's kernel: head sizes
-  // 64, 128 and 256 only.
-  if (p.mask && p.ms[2] != 0 && p.Tq > 1 && p.D != 64 && p.D != 128 && p.D != 256) return false;
   if (!aligned16(p.q) || !aligned16(p.k) || !aligned16(p.v) || !aligned16(p.out)) return false;
   for (int i = 0; i < 3; ++i)
     if (p.qs[i] % 8 || p.ks[i] % 8 || p.vs[i] % 8 || p.os[i] % 8) return false;  // 16-byte rows
@@ -376,10 +569,8 @@ int launch_flash_bf16(const SdpaParams& p, hipStream_t s) {
   // this file's kernel serves masks with a query-row stride, and head size
   // 256 in every form.  (With one query row the pipelined kernel's mask row
   // is that row.)
-  if (p.D == 256) return p.dtype == MFX_F16 ? launch_256<1>(p, s) : launch_256<0>(p, s);
-  if (!p.mask || p.ms[2] == 0 || p.Tq == 1) return launch_flash_bf16_pipe(p, s);
-  if (p.dtype == MFX_F16) return p.D == 128 ? launch_d<128, 1>(p, s) : launch_d<64, 1>(p, s);
-  return p.D == 128 ? launch_d<128, 0>(p, s) : launch_d<64, 0>(p, s);
+  if (p.D != 256 && (!p.mask || p.ms[2] == 0 || p.Tq == 1)) return launch_flash_bf16_pipe(p, s);
+  return p.dtype == MFX_F16 ? launch_d<1>(p, s) : launch_d<0>(p, s);
 }
 
 }  // namespace mfx

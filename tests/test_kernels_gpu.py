@@ -689,6 +689,76 @@ def test_sdpa_finite_mask_fully_masked_rows(cuda, nat, oracle, case, mdt):
     check_sdpa(out, select_semantics_ref(oracle, host(q), host(k), host(v), qs[-1] ** -0.5, keep), dt)
 
 
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("mdt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("D", [32, 64, 96, 128, 256])
+@pytest.mark.parametrize("tq,tk,form", [
+    (33, 8, "dense"), (65, 71, "dense"), (40, 64, "dense"), (130, 199, "dense"), (70, 130, "off_by_one"),
+    (40, 7, "dense"), (40, 90, "columns"), (40, 90, "row_constant"), (300, 333, "band")])
+def test_sdpa_query_varying_mask_runs(cuda, nat, oracle, dt, mdt, D, tq, tk, form):
+    """Masks that vary along query rows: read in runs of eight keys (rows that
+    start on and off a dword, ends short of a run and of a tile, a base one
+    element in) or element by element (fewer than eight keys, keys strided,
+    one value per row), and tiles with nothing visible, with causality."""
+    td = {"bf16": cuda.bfloat16, "f16": cuda.float16}[dt]
+    mt = {"f32": cuda.float32, "bf16": cuda.bfloat16, "f16": cuda.float16}[mdt]
+    q, k, v = make_qkv(cuda, 61, (2, 2, tq, D), (2, 1, tk, D), td)
+    rng = np.random.default_rng(62)
+    m = rng.standard_normal((2, 2, tq, tk))
+    m[rng.random(m.shape) < 0.2] = -np.inf
+    m[..., 0] = 0.5
+    causal = form == "dense" and tk == 71
+    if form == "columns":
+        maskd = dev(cuda, m, mt).transpose(2, 3).contiguous().transpose(2, 3)
+    elif form == "row_constant":
+        m[..., 1:] = m[..., :1] = rng.standard_normal((2, 2, tq, 1))
+        maskd = dev(cuda, m[..., :1], mt).expand(2, 2, tq, tk)
+        m = host(maskd)
+    elif form == "band":  # whole tiles off: keys more than 40 behind or ahead
+        i, j = np.arange(tq)[:, None], np.arange(tk)[None]
+        m = np.broadcast_to(np.where(np.abs(i - j) <= 40, m, -np.inf), m.shape).copy()
+        m[:, :, np.arange(tq), np.arange(tq)] = 0.25
+        maskd = dev(cuda, m, mt)
+    elif form == "off_by_one":
+        flat = cuda.zeros(m.size + 1, dtype=mt, device="cuda")
+        flat[1:] = dev(cuda, m, mt).flatten()
+        maskd = flat[1:].view(2, 2, tq, tk)
+    else:
+        maskd = dev(cuda, m, mt)
+    assert nat.sdpa_kernel_name(q, k, v, mask=maskd) == f"flash_{dt}_d{D}"
+    a = nat.sdpa(q, k, v, scale=D ** -0.5, mask=maskd, causal=causal)
+    ref = oracle.sdpa(host(q), host(k), host(v), D ** -0.5, causal=causal, mask=host(maskd))
+    check_sdpa(a, ref, "bf16")
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_sdpa_query_varying_mask_extremes(cuda, nat, oracle, D):
+    """A row of only -inf is NaN and its neighbours are not; a row whose first
+    visible key comes after tiles of -inf, and one that mixes -inf with the
+    lowest finite value, follow softmax."""
+    T = 200
+    q, k, v = make_qkv(cuda, 63, (1, 2, T, D), (1, 2, T, D), cuda.bfloat16)
+    m = np.zeros((1, 2, T, T))
+    m[0, 0, 5] = -np.inf
+    m[0, 0, 6, :150] = -np.inf
+    low = float(np.finfo(np.float32).min)
+    m[0, 1, 7, ::2] = -np.inf
+    m[0, 1, 7, 1::2] = low
+    m[0, 1, 8] = low
+    out = nat.sdpa(q, k, v, scale=D ** -0.5, mask=dev(cuda, m, cuda.float32))
+    o = host(out)
+    assert np.isnan(o[0, 0, 5]).all()
+    keep = m == 0
+    keep[0, 1, 7, 1::2] = True
+    keep[0, 1, 8] = True
+    ref = oracle.sdpa(host(q), host(k), host(v), D ** -0.5, mask=np.where(keep, 0.0, -np.inf))
+    vh = host(v)
+    ref[0, 1, 7] = vh[0, 1, 1::2].mean(0)
+    ref[0, 1, 8] = vh[0, 1].mean(0)
+    o[0, 0, 5] = ref[0, 0, 5] = 0
+    assert rel_inf(o, ref) <= BF16_REL_TOL
+
+
 def test_sdpa_decode_mfma_fully_masked_row_is_nan(cuda, nat):
     q, k, v = make_qkv(cuda, 24, (1, 4, 1, 64), (1, 2, 300, 64), cuda.bfloat16)
     mask = cuda.zeros(1, 4, 1, 300, device="cuda")
