@@ -220,8 +220,17 @@ def _lds_wait_errors(lines: list) -> list:
     return sorted(set(errors), key=lambda e: int(e.split()[1].rstrip(":")))
 
 
+# A "kill" note that ends one register in another's definition is a copy the
+# compiler dropped (seen here: a loop-carried value read from a register that
+# nothing wrote).
+_LOST_COPY = re.compile(r"kill: def \$([va])gpr(\d+)\S* killed \$([va])gpr(\d+)")
+
+
 def _check_lds_waits(src: Path, asm: str) -> None:
-    bad = []
+    bad = [f"a lost register copy: {m.group(0)}" for m in _LOST_COPY.finditer(asm)
+           if (m.group(1), m.group(2)) != (m.group(3), m.group(4))]
+    if bad:
+        raise RuntimeError(f"{src.name}:\n" + "\n".join(bad[:20]))
     name, body = None, []
     for ln, text in enumerate(asm.splitlines(), 1):
         m = re.match(r"^(_Z\S+):", text)

@@ -43,6 +43,7 @@
 #include <type_traits>
 
 #include "sdpa_elem.h"
+#include "sdpa_mask.h"
 #include "sdpa_tiles.h"
 
 #if defined(MFX_PHASE_TIMERS)
@@ -150,8 +151,9 @@ constexpr int kKvPf = 2;   // operand reads issued ahead of their MFMAs
 constexpr int kKvStages = 3;
 constexpr int kDkdvHeadGroup = 2;  // kv heads whose key blocks an XCD runs together
 
-template <int D, bool CAUSAL, bool MASK, int E>
+template <int D, bool CAUSAL, int MASKT, int E>
 __global__ __launch_bounds__(kNT, 1) void bwd_dkdv_mfma(SdpaBwdParams p) {
+  constexpr bool MASK = MASKT != 0;
   constexpr int TILE = kTile * D;    // elements of one Q or dO tile
   constexpr int TB = TILE * 2;       // its bytes
   constexpr int NK = D / 16;         // S (and dP) MFMAs per block
@@ -279,6 +281,43 @@ __global__ __launch_bounds__(kNT, 1) void bwd_dkdv_mfma(SdpaBwdParams p) {
   }
   const uint32_t la = base + LB + half * 16;  // lse | delta of rows 4*half ..
 
+  // The mask values of a block's 16 rows at this lane's key, all in flight
+  // from the end of the block before.  Loaded where they were used, each
+  // behind a branch on the type, they took more time than the products
+  // (sdpa_mask.h).
+  // (As loaded: 16-bit types convert at their use.)
+  uint32_t mv[MASK ? 16 : 1];
+  using MElem = std::conditional_t<MASKT == 2 || MASKT == 3, uint16_t, uint32_t>;
+  const int64_t mcol = MASK ? b * p.ms[0] + (int64_t)hk * G * p.ms[1] + (int64_t)min(key, Tk - 1) * p.ms[3] : 0;
+  auto mask_load = [&](int t, auto mt_tag) __attribute__((always_inline)) {
+    constexpr int MT = decltype(mt_tag)::value;
+    if constexpr (MASK) {
+      const int q = tile_q(t) * kTile + MT * 32;
+      const int64_t head = mcol + (int64_t)tile_head(t) * p.ms[1];
+      if (q + 32 <= Tq && MASKT != kAnyMask) {
+        const MElem* at = static_cast<const MElem*>(p.mask) + head + (int64_t)(q + half * 4) * p.ms[2];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          mv[i] = *at;
+          at += (i & 3) == 3 ? 5 * p.ms[2] : p.ms[2];
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int64_t off = head + (int64_t)min(q + (i >> 2) * 8 + half * 4 + (i & 3), Tq - 1) * p.ms[2];
+          if constexpr (MASKT == kAnyMask) mv[i] = __float_as_uint(load_mask(p.mask, p.mask_dtype, off));
+          else mv[i] = static_cast<const MElem*>(p.mask)[off];
+        }
+      }
+    }
+  };
+
+  auto mask_val = [&](int i) {
+    if constexpr (MASKT == 2) return __uint_as_float(mv[i] << 16);
+    else if constexpr (MASKT == 3) return f16_lo(mv[i]);
+    else return __uint_as_float(mv[i]);
+  };
+
   f32x16 s, dp;         // S and dP of the block in flight
   u32x4 pd[2][2][2];    // [block parity][P | dS][16-query step]: bf16 pairs
 
@@ -314,8 +353,8 @@ __global__ __launch_bounds__(kNT, 1) void bwd_dkdv_mfma(SdpaBwdParams p) {
 
   // Y | V: dV^T += dO^T P and dK^T += Q^T dS of block (PS, PM) (P and dS in
   // pd[PM]), with (VAL) the P / dS of block (ST, MT) -- from s and dp -- into
-  // pd[MT] between the MFMAs.  q0b: the block's first query; g: its head.
-  auto YV = [&](auto ps_tag, auto pm_tag, auto st_tag, auto mt_tag, auto edge_tag, auto val_tag, int q0b, int g)
+  // pd[MT] between the MFMAs.  q0b: the block's first query.
+  auto YV = [&](auto ps_tag, auto pm_tag, auto st_tag, auto mt_tag, auto edge_tag, auto val_tag, int q0b)
       __attribute__((always_inline)) {
     constexpr int PS = decltype(ps_tag)::value, PM = decltype(pm_tag)::value;
     constexpr int ST = decltype(st_tag)::value, MT = decltype(mt_tag)::value;
@@ -377,12 +416,7 @@ __global__ __launch_bounds__(kNT, 1) void bwd_dkdv_mfma(SdpaBwdParams p) {
             const int i = 2 * k + u, r = i >> 2, e = i & 3;
             const int q = q0b + r * 8 + half * 4 + e;
             float x = fmaf(sv[u], sl2, -lq[r][e]);
-            if constexpr (MASK) {
-              if (q < Tq && key < Tk)
-                x += mask_log2(load_mask(p.mask, p.mask_dtype,
-                                        b * p.ms[0] + (int64_t)(hk * G + g) * p.ms[1] + (int64_t)q * p.ms[2] +
-                                            (int64_t)key * p.ms[3]));
-            }
+            if constexpr (MASK) x += mask_log2(mask_val(i));
             pr[u] = __builtin_amdgcn_exp2f(x);
             if constexpr (EDGE) {
               if (q >= Tq || (CAUSAL && key > q)) pr[u] = 0.f;
@@ -402,15 +436,16 @@ __global__ __launch_bounds__(kNT, 1) void bwd_dkdv_mfma(SdpaBwdParams p) {
   // Block (ST, MT) of tile t after block (PS, PM): X, then Y | V.
   auto step = [&](int t, auto ps_tag, auto pm_tag, auto st_tag, auto mt_tag) __attribute__((always_inline)) {
     constexpr int MT = decltype(mt_tag)::value;
-    const int g = tile_head(t), q0b = tile_q(t) * kTile + MT * 32;
+    const int q0b = tile_q(t) * kTile + MT * 32;
     PHASE(fence(); const unsigned c0 = ph_now(); fence();)
     X(st_tag, mt_tag);
     PHASE(fence(); const unsigned c1 = ph_now(); fence();)
     const bool edge = (q0b + 32 > Tq) || (CAUSAL && q0b < kw + 31);
     if (edge)
-      YV(ps_tag, pm_tag, st_tag, mt_tag, std::true_type{}, std::true_type{}, q0b, g);
+      YV(ps_tag, pm_tag, st_tag, mt_tag, std::true_type{}, std::true_type{}, q0b);
     else
-      YV(ps_tag, pm_tag, st_tag, mt_tag, std::false_type{}, std::true_type{}, q0b, g);
+      YV(ps_tag, pm_tag, st_tag, mt_tag, std::false_type{}, std::true_type{}, q0b);
+    if (MASK && (MT == 0 || t + 1 < ntiles)) mask_load(t + MT, std::integral_constant<int, 1 - MT>{});
     PHASE(fence(); const unsigned c2 = ph_now(); ph_add(kPhX, c1 - c0); ph_add(kPhYV, c2 - c1);
           ph_add(kPhBlocks, 1u); ph_add(kPhEdges, edge ? 1u : 0u); fence();)
   };
@@ -441,6 +476,7 @@ __global__ __launch_bounds__(kNT, 1) void bwd_dkdv_mfma(SdpaBwdParams p) {
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int k = 0; k < 2; ++k) pd[1][i][k] = u32x4{0u, 0u, 0u, 0u};
+    mask_load(0, I0{});
     tile(0, I0{}, I0{});
     for (int t = 1;; t += 3) {
       if (t >= ntiles) break;
@@ -454,11 +490,11 @@ __global__ __launch_bounds__(kNT, 1) void bwd_dkdv_mfma(SdpaBwdParams p) {
     PHASE(fence(); const unsigned cl = ph_now(); fence();)
     const int ls = (ntiles - 1) % kKvStages;
     if (ls == 0)
-      YV(I0{}, I1{}, I0{}, I0{}, std::false_type{}, std::false_type{}, 0, 0);
+      YV(I0{}, I1{}, I0{}, I0{}, std::false_type{}, std::false_type{}, 0);
     else if (ls == 1)
-      YV(I1{}, I1{}, I0{}, I0{}, std::false_type{}, std::false_type{}, 0, 0);
+      YV(I1{}, I1{}, I0{}, I0{}, std::false_type{}, std::false_type{}, 0);
     else
-      YV(I2{}, I1{}, I0{}, I0{}, std::false_type{}, std::false_type{}, 0, 0);
+      YV(I2{}, I1{}, I0{}, I0{}, std::false_type{}, std::false_type{}, 0);
     PHASE(fence(); ph_add(kPhLast, ph_now() - cl); fence();)
   }
 
@@ -523,8 +559,10 @@ __global__ __launch_bounds__(kNT, 1) void bwd_dkdv_mfma(SdpaBwdParams p) {
 // fragment pairs, transposed K fragment pairs).
 constexpr int kDqPf = 2;
 
-template <int D, bool CAUSAL, bool MASK, int E>
-__global__ __launch_bounds__(kNT, 2) void bwd_dq_mfma(SdpaBwdParams p) {
+// Two workgroups per CU, except D = 128 with mask runs in registers (~300).
+template <int D, bool CAUSAL, int MASKT, int E>
+__global__ __launch_bounds__(kNT, D == 128 && MASKT != 0 && MASKT != kAnyMask ? 1 : 2) void bwd_dq_mfma(SdpaBwdParams p) {
+  constexpr bool MASK = MASKT != 0, RUNS = MASK && MASKT != kAnyMask;
   constexpr int TILE = kTile * D;  // elements of one K or V tile
   constexpr int TB = TILE * 2;     // its bytes
   constexpr int NK = D / 16;       // S (and dP) MFMAs per 32-key block
@@ -612,24 +650,40 @@ __global__ __launch_bounds__(kNT, 2) void bwd_dq_mfma(SdpaBwdParams p) {
   // LDS byte addresses of the operand reads; the stage, the 32-key block and
   // the 16-key step are immediate offsets.
   const uint32_t base = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)smem;
+  // Row r of a 32-key block is key r; with a mask in runs, r with bits 2 and
+  // 3 swapped, so that a lane's scores of a 16-key step belong to eight
+  // consecutive keys, half*8 + (0..7).
+  constexpr int RH = RUNS ? 8 : 4, RS = 12 - RH;  // key of slot e: RH*half + e, slot 4 + e: that + RS
   uint32_t ra[D / 16];  // row l32 of a 32-key block, feature chunk kk
   {
-    const int rsw = tile_swz<D>(l32);
+    const int r = RUNS ? (l32 & ~12) | (l32 & 4) << 1 | (l32 & 8) >> 1 : l32;
+    const int rsw = tile_swz<D>(r);
 #pragma unroll
-    for (int kk = 0; kk < D / 16; ++kk) ra[kk] = base + (uint32_t)((l32 * D + ((kk * 2 + half) ^ rsw) * 8) * 2);
+    for (int kk = 0; kk < D / 16; ++kk) ra[kk] = base + (uint32_t)((r * D + ((kk * 2 + half) ^ rsw) * 8) * 2);
   }
-  uint32_t ta[D / 32][2];  // transposing reads of K (the order of TrReader)
+  uint32_t ta[D / 32][2];  // transposing reads of K
   {
     const int tj = lane & 15, tg = (lane >> 4) & 1;
-    const int r = 4 * half + (tj >> 2);
-    const int sw = tile_swz<D>(r), sw8 = tile_swz<D>(r + 8);
+    const int r = RH * half + (tj >> 2);
+    const int sw = tile_swz<D>(r), sw2 = tile_swz<D>(r + RS);
     const int chunk = tg * 2 + ((tj & 3) >> 1), sub = (tj & 1) * 4;
 #pragma unroll
     for (int dt = 0; dt < D / 32; ++dt) {
       ta[dt][0] = base + (uint32_t)((r * D + sub + ((dt * 4 + chunk) ^ sw) * 8) * 2);
-      ta[dt][1] = base + (uint32_t)(((r + 8) * D + sub + ((dt * 4 + chunk) ^ sw8) * 8) * 2);
+      ta[dt][1] = base + (uint32_t)(((r + RS) * D + sub + ((dt * 4 + chunk) ^ sw2) * 8) * 2);
     }
   }
+  // The block's mask values, loaded while the block before ran.
+  using Run = MaskRun<RUNS ? MASKT : 1>;
+  Run mk[2];
+  const int64_t moff = MASK ? b * p.ms[0] + (int64_t)h * p.ms[1] + (int64_t)min(qi, Tq - 1) * p.ms[2] : 0;
+  const auto* mrow = static_cast<const typename Run::Elem*>(p.mask) + moff;
+  const bool odd = RUNS && mask_runs_odd<RUNS ? MASKT : 1>(p);
+  auto mask_load = [&](Run (&to)[2], int k0) __attribute__((always_inline)) {
+    to[0].load(mrow, k0 + half * 8, Tk, odd);
+    to[1].load(mrow, k0 + 16 + half * 8, Tk, odd);
+  };
+  if constexpr (RUNS) mask_load(mk, 0);
 
   // One 32-key block (MT) of the tile in stage ST:
   //   S^T = K Q^T and dP^T = V dO^T, their MFMAs alternating, K and V row
@@ -641,6 +695,15 @@ __global__ __launch_bounds__(kNT, 2) void bwd_dq_mfma(SdpaBwdParams p) {
     constexpr int KO = 2 * ST * TB + MT * 32 * D * 2;  // K rows of this block
     constexpr int VO = KO + TB;                        // V rows
     constexpr int KT = 2 * ST * TB;                    // K tile (transposing reads)
+    const int k0 = kb + MT * 32;
+    bool off = false;
+    if constexpr (RUNS) {
+      const bool ragged = EDGE && k0 + 32 > Tk;
+      if (odd || ragged) place_runs(mk, mrow, k0 + half * 8, Tk, odd, ragged);
+      off = runs_all_off(mk);  // every dS is zero
+    }
+    bf16x8 db[2];
+    if (!off) {
     bf16x8 kf[NK], vf[NK];
     auto rd = [&](auto j_tag) {
       constexpr int j = decltype(j_tag)::value;
@@ -666,18 +729,13 @@ __global__ __launch_bounds__(kNT, 2) void bwd_dq_mfma(SdpaBwdParams p) {
         dp = mfma16<E>(vf[j], gf[j], dp);
       fence();
     });
-    bf16x8 db[2];
     float dsv[16];  // f16: dS before its rounding, packed by pairs below
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const int key = kb + MT * 32 + (i >> 2) * 8 + half * 4 + (i & 3);
+      const int key = RUNS ? k0 + (i >> 3) * 16 + half * 8 + (i & 7) : k0 + (i >> 2) * 8 + half * 4 + (i & 3);
       float x = s[i] * sl2;
-      if constexpr (MASK) {
-        if (qi < Tq && key < Tk)
-          x += mask_log2(load_mask(p.mask, p.mask_dtype,
-                                  b * p.ms[0] + (int64_t)h * p.ms[1] + (int64_t)qi * p.ms[2] +
-                                      (int64_t)key * p.ms[3]));
-      }
+      if constexpr (RUNS) x += mask_log2(mk[i >> 3].get(i & 7));
+      else if constexpr (MASK) x += mask_log2(load_mask(p.mask, p.mask_dtype, moff + min(key, Tk - 1) * p.ms[3]));
       float pr = __builtin_amdgcn_exp2f(x - lse);
       if constexpr (EDGE) {
         if (key >= Tk || (CAUSAL && key > qi)) pr = 0.f;
@@ -694,6 +752,8 @@ __global__ __launch_bounds__(kNT, 2) void bwd_dq_mfma(SdpaBwdParams p) {
         db[h2] = f32_frag_f16(t);
       }
     }
+    }
+    if (off) return;
     // dQ MFMA j: d-block j % (D/32), 16-key step j / (D/32) of this block.
     s16x4 tr[NT][2];
     auto rdt = [&](auto j_tag) {
@@ -724,10 +784,16 @@ __global__ __launch_bounds__(kNT, 2) void bwd_dq_mfma(SdpaBwdParams p) {
       const int k0r = kb + MT * 32;
       if (k0r >= Tk || (CAUSAL && k0r > q0 + 31)) return;  // nothing of this block is visible
       const bool edge = (k0r + 32 > Tk) || (CAUSAL && k0r + 31 > q0);
+      // (Unconditional: past the last block it re-reads the row's end.)
+      Run next[2];
+      if constexpr (RUNS) mask_load(next, k0r + 32);
       if (edge)
         block(st_tag, mt_tag, kb, std::true_type{});
       else
         block(st_tag, mt_tag, kb, std::false_type{});
+      if constexpr (RUNS)
+#pragma unroll
+        for (int g = 0; g < 2; ++g) mk[g] = next[g];
     });
   };
 
@@ -758,21 +824,30 @@ __global__ __launch_bounds__(kNT, 2) void bwd_dq_mfma(SdpaBwdParams p) {
   }
 }
 
-template <int D, bool CAUSAL, bool MASK, int E>
+template <int D, bool CAUSAL, int MT, int E>
 int launch_t(const SdpaBwdParams& p, hipStream_t s) {
   const int64_t q_blocks = (int64_t)p.B * p.Hq * ((p.Tq + kRows - 1) / kRows);
-  hipLaunchKernelGGL((bwd_dq_mfma<D, CAUSAL, MASK, E>), dim3((unsigned)q_blocks), dim3(kNT), 0, s, p);
+  hipLaunchKernelGGL((bwd_dq_mfma<D, CAUSAL, MT, E>), dim3((unsigned)q_blocks), dim3(kNT), 0, s, p);
   if (int rc = launch_status("bwd_dq_mfma")) return rc;
   const int64_t kv_blocks = (int64_t)p.B * p.Hkv * ((p.Tk + kRows - 1) / kRows);
-  hipLaunchKernelGGL((bwd_dkdv_mfma<D, CAUSAL, MASK, E>), dim3((unsigned)kv_blocks), dim3(kNT), 0, s, p);
+  hipLaunchKernelGGL((bwd_dkdv_mfma<D, CAUSAL, MT, E>), dim3((unsigned)kv_blocks), dim3(kNT), 0, s, p);
   return launch_status("bwd_dkdv_mfma");
+}
+
+template <int D, bool CAUSAL, int E>
+int launch_m(const SdpaBwdParams& p, hipStream_t s) {
+  switch (mask_run_code(p)) {
+    case 0: return launch_t<D, CAUSAL, 0, E>(p, s);
+    case 1: return launch_t<D, CAUSAL, 1, E>(p, s);
+    case 2: return launch_t<D, CAUSAL, 2, E>(p, s);
+    case 3: return launch_t<D, CAUSAL, 3, E>(p, s);
+    default: return launch_t<D, CAUSAL, kAnyMask, E>(p, s);
+  }
 }
 
 template <int D, int E>
 int launch_d(const SdpaBwdParams& p, hipStream_t s) {
-  const bool m = p.mask != nullptr;
-  if (p.causal) return m ? launch_t<D, true, true, E>(p, s) : launch_t<D, true, false, E>(p, s);
-  return m ? launch_t<D, false, true, E>(p, s) : launch_t<D, false, false, E>(p, s);
+  return p.causal ? launch_m<D, true, E>(p, s) : launch_m<D, false, E>(p, s);
 }
 
 bool aligned16(const void* ptr) { return ((uintptr_t)ptr & 15) == 0; }

@@ -34,6 +34,7 @@
 #include <type_traits>
 
 #include "sdpa_elem.h"
+#include "sdpa_mask.h"
 #include "sdpa_tiles.h"
 
 namespace mfx {
@@ -54,93 +55,11 @@ using tiles::fence;
 template <int D>
 using TileLoader = tiles::TileLoader<D, kBN, kNT / 64>;
 
-// One lane's mask values of eight consecutive keys of its query row, as raw
-// bits.  MT: mask_code of the mask's type.
-//
-// Loading whole runs is what makes this kernel fast: one element at a time
-// behind a branch on the type, each load waited for alone, a
-// [1,16,1999,1999] bf16 bias took 1045 us a call on [4,16,1999,128] GQA;
-// in runs, a tile's all in flight a tile ahead, 221 (179 with 2048 keys,
-// against 129 without a mask: what is left is the mask's own vector work
-// and its loads, 32 rows of 32 bytes each).
-template <int MT>
-struct MaskRun {
-  using Elem = std::conditional_t<MT == 1, uint32_t, uint16_t>;
-  static constexpr int NW = MT == 1 ? 8 : 4;  // dwords
-  // -inf throughout, which removes the keys.
-  static constexpr uint32_t kOff = MT == 1 ? 0xFF800000u : MT == 2 ? 0xFF80FF80u : 0xFC00FC00u;
-  uint32_t w[NW + (MT != 1)];
-
-  // Keys key .. key + 7 of the row at `row` (key stride 1, at least eight
-  // keys) as 16-byte loads on any 4-byte boundary.  A run that would pass the
-  // row's end is moved back inside it; shift() undoes that.
-  //
-  // odd: some run may start on an odd 16-bit element.  Loads off a 4-byte
-  // boundary are slow (259 against 179 us with a 1999- and a 2048-key bias),
-  // so such runs load the five dwords that hold them and align() moves them
-  // into place.  (No dword without a byte of the run is touched.)
-  __device__ __forceinline__ void load(const Elem* row, int key, int Tk, bool odd) {
-    load(row + min(key, Tk - 8), odd);
-  }
-  __device__ __forceinline__ void load(const Elem* at, bool odd) {
-    typedef uint32_t run_t __attribute__((ext_vector_type(4), aligned(4)));
-    const char* from = reinterpret_cast<const char*>(reinterpret_cast<uintptr_t>(at) & ~uintptr_t(3));
-#pragma unroll
-    for (int c = 0; c < NW / 4; ++c) {
-      const run_t v = *reinterpret_cast<const run_t*>(from + c * 16);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) w[c * 4 + j] = v[j];
-    }
-    if constexpr (MT != 1)
-      if (odd) w[4] = *reinterpret_cast<const uint32_t*>(from + 12 + 2 * (reinterpret_cast<uintptr_t>(at) & 2));
-  }
-  // After an odd load; par: 1 when the run began on an odd element.
-  __device__ __forceinline__ void align(uint32_t par) {
-    if constexpr (MT != 1)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) w[j] = __builtin_amdgcn_alignbit(w[j + 1], w[j], par * 16);
-  }
-  // At a ragged end: moves the run's first valid value back to slot 0 (the
-  // slots past Tk keep something; the caller masks them).
-  __device__ __forceinline__ void shift(int key, int Tk) {
-    const int d = key - min(key, Tk - 8);
-    if constexpr (MT == 1) {
-#pragma unroll
-      for (int by = 1; by < 8; by *= 2)
-#pragma unroll
-        for (int j = 0; j + by < 8; ++j) {
-          const uint32_t a = w[j], b = w[j + by];
-          w[j] = (d & by) ? b : a;
-        }
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t a = w[j], b = w[(j + 1) & 3];
-        w[j] = (d & 1) ? a >> 16 | b << 16 : a;
-      }
-#pragma unroll
-      for (int by = 1; by < 4; by *= 2)
-#pragma unroll
-        for (int j = 0; j + by < 4; ++j) {
-          const uint32_t a = w[j], b = w[j + by];
-          w[j] = (d & 2 * by) ? b : a;
-        }
-    }
-  }
-  __device__ __forceinline__ float get(int j) const {
-    if constexpr (MT == 1) return __uint_as_float(w[j]);
-    else if constexpr (MT == 2) return __uint_as_float((j & 1) ? w[j >> 1] & 0xFFFF0000u : w[j >> 1] << 16);
-    else return (j & 1) ? f16_hi(w[j >> 1]) : f16_lo(w[j >> 1]);
-  }
-};
-
 // D: LDS row width (64, 128 or 256), DV <= D: the head size.  MT: the mask's
 // type (mask_code) read in runs; kAnyMask: any type and key stride, read
 // element by element; 0: no mask (D = 256 only).
 // D = 256: one workgroup per CU (four 32 KB tiles; O, Q and S of a wavefront
 // take ~300 registers).
-constexpr int kAnyMask = 4;
-
 template <int D, int DV, int MT, int E>
 __global__ __launch_bounds__(kNT, D > 128 ? 1 : 2) void flash_bf16_kernel(SdpaParams p) {
   __shared__ __attribute__((aligned(16))) bf16 k0[kBN * D];
@@ -202,12 +121,7 @@ __global__ __launch_bounds__(kNT, D > 128 ? 1 : 2) void flash_bf16_kernel(SdpaPa
   Run mk[AHEAD ? kKS : 1];
   const int64_t moff = MASK ? b * p.ms[0] + h * p.ms[1] + (int64_t)min(qi, Tq - 1) * p.ms[2] : 0;
   const auto* mrow = static_cast<const typename Run::Elem*>(p.mask) + moff;
-  // (16-bit masks: a row, or the run at a ragged row's end, may start off a
-  // dword; row_par: this lane's row does.)
-  const bool odd =
-      RUNS && MT != 1 &&
-      (((reinterpret_cast<uintptr_t>(p.mask) >> 1) | p.ms[0] | p.ms[1] | p.ms[2] | Tk) & 1) != 0;
-  const uint32_t row_par = (uint32_t)(reinterpret_cast<uintptr_t>(mrow) >> 1) & 1;
+  const bool odd = RUNS && mask_runs_odd<RUNS ? MT : 1>(p);
   auto mask_load = [&](int kb) __attribute__((always_inline)) {
     if (kb + kBN <= Tk) {
       const auto* at = mrow + (kb + half * 8);
@@ -217,22 +131,6 @@ __global__ __launch_bounds__(kNT, D > 128 ? 1 : 2) void flash_bf16_kernel(SdpaPa
 #pragma unroll
       for (int g = 0; g < kKS; ++g) mk[AHEAD ? g : 0].load(mrow, kb + g * 16 + half * 8, Tk, odd);
     }
-  };
-  // The loaded runs of a tile put in place: `ragged` when it passes Tk.
-  auto run_place = [&](Run& run, int key, bool ragged) __attribute__((always_inline)) {
-    if (odd) run.align(row_par ^ (ragged ? min(key, Tk - 8) & 1 : 0));
-    if (ragged) run.shift(key, Tk);
-  };
-  // Whether every lane's every value is -inf.  The first value decides for
-  // nearly every tile that is not.
-  auto mask_all_off = [&]() __attribute__((always_inline)) {
-    if (__ballot(mk[0].w[0] != Run::kOff)) return false;
-    uint32_t d = 0;
-#pragma unroll
-    for (int g = 0; g < kKS; ++g)
-#pragma unroll
-      for (int j = 0; j < Run::NW; ++j) d |= mk[AHEAD ? g : 0].w[j] ^ Run::kOff;
-    return __ballot(d != 0) == 0;
   };
   if constexpr (AHEAD) mask_load(0);
 
@@ -282,14 +180,13 @@ __global__ __launch_bounds__(kNT, D > 128 ? 1 : 2) void flash_bf16_kernel(SdpaPa
     const char* kb8 = reinterpret_cast<const char*>(kl);
     const char* vb8 = reinterpret_cast<const char*>(vl);
     const bool more = kb + kBN < kv_end;
+    // Nothing visible: a band or block mask's tiles outside it.
+    bool off = false;
     if constexpr (AHEAD) {
       const bool ragged = EDGE && kb + kBN > Tk;
-      if (odd || ragged)
-#pragma unroll
-        for (int g = 0; g < kKS; ++g) run_place(mk[g], kb + g * 16 + half * 8, ragged);
+      if (odd || ragged) place_runs(mk, mrow, kb + half * 8, Tk, odd, ragged);
+      off = runs_all_off(mk);
     }
-    // Nothing visible: a band or block mask's tiles outside it.
-    const bool off = AHEAD && mask_all_off();
     f32x16 s[kMT];
     float mx = -INFINITY;
     if (!off) {
@@ -341,7 +238,7 @@ __global__ __launch_bounds__(kNT, D > 128 ? 1 : 2) void flash_bf16_kernel(SdpaPa
             if ((i & 7) == 0) {
               fence();
               run.load(mrow, key, Tk, odd);
-              run_place(run, key, EDGE && kb + kBN > Tk);
+              place_runs(mk, mrow, key, Tk, odd, EDGE && kb + kBN > Tk);
             }
           float m = run.get(i & 7);
           if constexpr (AHEAD) {
@@ -521,11 +418,11 @@ int launch_t(const SdpaParams& p, hipStream_t s) {
 
 template <int D, int DV, int E>
 int launch_m(const SdpaParams& p, hipStream_t s) {
-  if (p.ms[3] != 1 || p.Tk < 8) return launch_t<D, DV, kAnyMask, E>(p, s);
-  switch (mask_code(p.mask_dtype)) {
+  switch (mask_run_code(p)) {
     case 1: return launch_t<D, DV, 1, E>(p, s);
     case 2: return launch_t<D, DV, 2, E>(p, s);
-    default: return launch_t<D, DV, 3, E>(p, s);
+    case 3: return launch_t<D, DV, 3, E>(p, s);
+    default: return launch_t<D, DV, kAnyMask, E>(p, s);
   }
 }
 

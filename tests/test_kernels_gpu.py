@@ -864,6 +864,39 @@ def test_sdpa_bwd_padded_btnh_mask_and_residuals(cuda, nat, oracle, D):
         assert cuda.equal(a, b)
 
 
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("mdt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("D,tq,tk,form", [(64, 33, 8, "dense"), (128, 65, 71, "dense"), (128, 130, 199, "off_by_one"),
+                                          (64, 97, 96, "columns"), (128, 40, 7, "dense"), (128, 150, 150, "band"),
+                                          (64, 150, 150, "causal")])
+def test_sdpa_bwd_query_varying_mask_runs(cuda, nat, oracle, dt, mdt, D, tq, tk, form):
+    """Masked 16-bit backward with GQA: mask runs on and off a dword, short of
+    a run, strided keys, blocks with nothing visible, causality."""
+    td = {"bf16": cuda.bfloat16, "f16": cuda.float16}[dt]
+    mt = {"f32": cuda.float32, "bf16": cuda.bfloat16, "f16": cuda.float16}[mdt]
+    q, k, v = make_qkv(cuda, 71, (2, 4, tq, D), (2, 2, tk, D), td)
+    rng = np.random.default_rng(72)
+    g = dev(cuda, rng.standard_normal((2, 4, tq, D)), td)
+    m = rng.standard_normal((2, 4, tq, tk))
+    m[rng.random(m.shape) < 0.2] = -np.inf
+    m[..., 0] = 0.5
+    if form == "band":
+        i, j = np.arange(tq)[:, None], np.arange(tk)[None]
+        m = np.where(np.abs(i - j) <= 20, np.where(i == j, 0.25, m), -np.inf)
+    maskd = dev(cuda, m, mt)
+    if form == "columns":
+        maskd = maskd.transpose(2, 3).contiguous().transpose(2, 3)
+    if form == "off_by_one":
+        flat = cuda.zeros(m.size + 1, dtype=mt, device="cuda")
+        flat[1:] = maskd.flatten()
+        maskd = flat[1:].view(2, 4, tq, tk)
+    assert nat.sdpa_bwd_kernel_name(q, k, v, mask=maskd) == f"mfma_{dt}_d{D}"
+    causal = form == "causal"
+    grads = nat.sdpa_bwd(q, k, v, g, causal=causal, mask=maskd)
+    refs = oracle.sdpa_bwd(host(q), host(k), host(v), host(g), D ** -0.5, causal=causal, mask=host(maskd))
+    check_grads(grads, refs, "bf16")
+
+
 def test_sdpa_bwd_odd_head_size_generic(cuda, nat, oracle):
     grads, refs = bwd_case(cuda, nat, oracle, 43, (1, 3, 50, 80), (1, 3, 70, 80), "bf16", causal=True,
                            vshape=(1, 3, 70, 48))
