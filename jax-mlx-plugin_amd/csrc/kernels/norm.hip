@@ -3,8 +3,9 @@
 //
 // A row is owned by 16 or 64 lanes of one wavefront (rows up to 1024
 // 16-byte vectors, i.e. 4096 f32 / 8192 bf16 or f16 elements) or by a 256-thread
-// workgroup (up to 4096 vectors); longer or unaligned rows take a looped
-// fallback.  Each element is read from HBM once and written once -- the HBM
+// workgroup (up to 4096 vectors); unaligned rows and rows of up to 64 Ki
+// elements take row_kernel_any (up to 1024 threads a row), longer ones a
+// looped fallback.  Each element is read from HBM once and written once -- the HBM
 // roofline's algorithmic traffic.
 #include "rowvec.h"
 
@@ -145,9 +146,150 @@ __global__ __launch_bounds__(kBlock) void row_kernel(
   }
 }
 
-// Fallback for rows that are not 16-byte vectorisable or longer than the
-// register-resident variants: one workgroup per row, scalar strided loops,
-// three passes over the row.
+// Runs of VEC elements from e on, of a row of n at any alignment: 16 bytes at
+// a time (a dword-aligned 16-byte load costs what an aligned one does), the
+// row's last, partial run element by element.
+template <typename T, int VEC>
+__device__ __forceinline__ void load_run(const T* row, int e, int n, float fill, float (&out)[VEC]) {
+  if (e + VEC <= n) {
+    if constexpr (sizeof(T) == 4) {
+      typedef float run_t __attribute__((ext_vector_type(4), aligned(4)));
+#pragma unroll
+      for (int c = 0; c < VEC / 4; ++c) {
+        const run_t r = *reinterpret_cast<const run_t*>(row + e + c * 4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) out[c * 4 + j] = r[j];
+      }
+    } else {
+      typedef uint32_t run_t __attribute__((ext_vector_type(VEC / 2), aligned(2)));
+      const run_t r = *reinterpret_cast<const run_t*>(row + e);
+#pragma unroll
+      for (int j = 0; j < VEC / 2; ++j) {
+        if constexpr (std::is_same<T, _Float16>::value) {
+          out[2 * j] = f16_lo(r[j]);
+          out[2 * j + 1] = f16_hi(r[j]);
+        } else {
+          out[2 * j] = __uint_as_float(r[j] << 16);
+          out[2 * j + 1] = __uint_as_float(r[j] & 0xffff0000u);
+        }
+      }
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) out[j] = e + j < n ? to_f32(row[e + j]) : fill;
+  }
+}
+
+template <typename T, int VEC>
+__device__ __forceinline__ void store_run(T* row, int e, int n, const float (&v)[VEC]) {
+  if (e + VEC <= n) {
+    if constexpr (sizeof(T) == 4) {
+      typedef float run_t __attribute__((ext_vector_type(4), aligned(4)));
+      *reinterpret_cast<run_t*>(row + e) = run_t{v[0], v[1], v[2], v[3]};
+    } else {
+      typedef uint32_t run_t __attribute__((ext_vector_type(4), aligned(2)));
+      const typename Vec16<T>::type w = pack16<T>(v);
+      *reinterpret_cast<run_t*>(row + e) = run_t{w.x, w.y, w.z, w.w};
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < VEC; ++j)
+      if (e + j < n) row[e + j] = from_f32<T>(v[j]);
+  }
+}
+
+// row_kernel for rows of any length and alignment that fit the registers of
+// LANES threads (64, 256, or a 1024-thread workgroup): the row read once, in
+// runs of 16 bytes, parameters read in the epilogue (at 1024 threads there
+// are 128 registers a thread).
+//
+// Bound by HBM: log-softmax of [4096, 32003] f32 (rows off 16 bytes; 1.05 GB)
+// takes 195 us (5.4 TB/s), against 491 us in the looped kernel, which reads
+// such a row three times, one element per load; of [40311, 310] f16 19 us
+// against 50.  LayerNorm of [4096, 32003]: 244 us against 727.
+template <typename T, typename PT, int LANES, int NV, RowOp OP>
+__global__ __launch_bounds__(LANES > kBlock ? LANES : kBlock) void row_kernel_any(
+    const T* __restrict__ x, T* __restrict__ y, const PT* __restrict__ gamma, const PT* __restrict__ beta,
+    int64_t rows, int n, int64_t xs, int64_t ys, float eps) {
+  constexpr int VEC = Vec16<T>::N;
+  constexpr int BLOCK = LANES > kBlock ? LANES : kBlock;
+  __shared__ float lds[BLOCK / 64];
+  const int lane = threadIdx.x % LANES;
+  const int64_t row = (int64_t)blockIdx.x * (BLOCK / LANES) + threadIdx.x / LANES;
+  const bool row_ok = row < rows;
+  const T* xr = x + (row_ok ? row : 0) * xs;
+  constexpr float kFill = is_softmax(OP) ? -INFINITY : 0.f;
+  float v[NV][VEC];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) load_run<T, VEC>(xr, (i * LANES + lane) * VEC, row_ok ? n : 0, kFill, v[i]);
+
+  const float inv_n = 1.0f / (float)n;
+  float scale = 0.f, shift = 0.f;
+  if constexpr (is_softmax(OP)) {
+    float m = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) m = fmaxf(m, v[i][j]);
+    m = row_reduce<LANES, true>(m, lds);
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) {
+        const float e = __expf(v[i][j] - m);
+        if constexpr (OP == RowOp::kSoftmax) v[i][j] = e;
+        s += e;
+      }
+    s = row_reduce<LANES, false>(s, lds);
+    if constexpr (OP == RowOp::kSoftmax) scale = 1.0f / s;
+    else shift = m + logf(s);
+  } else {
+    if constexpr (OP == RowOp::kLayerNorm) {
+      float s = 0.f;
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) s += v[i][j];
+      shift = row_reduce<LANES, false>(s, lds) * inv_n;
+    }
+    float q = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) {
+        const float d = v[i][j] - shift;
+        q += (i * LANES + lane) * VEC + j < n ? d * d : 0.f;
+      }
+    scale = rsqrtf(row_reduce<LANES, false>(q, lds) * inv_n + eps);
+  }
+  if (!row_ok) return;
+  T* yr = y + row * ys;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int e = (i * LANES + lane) * VEC;
+    if (e >= n) continue;
+    float o[VEC];
+    if constexpr (is_softmax(OP)) {
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) o[j] = OP == RowOp::kSoftmax ? v[i][j] * scale : v[i][j] - shift;
+    } else {
+      float g[VEC], b[VEC];
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) g[j] = 1.f, b[j] = 0.f;
+      if (gamma) load_run<PT, VEC>(gamma, e, n, 1.f, g);
+      if (OP == RowOp::kLayerNorm && beta) load_run<PT, VEC>(beta, e, n, 0.f, b);
+#pragma unroll
+      for (int j = 0; j < VEC; ++j)
+        o[j] = OP == RowOp::kLayerNorm ? fmaf((v[i][j] - shift) * scale, g[j], b[j]) : v[i][j] * scale * g[j];
+    }
+    store_run<T, VEC>(yr, e, n, o);
+  }
+}
+
+// Fallback for rows longer than the register-resident variants (and
+// parameters of a type those do not take): one workgroup per row, scalar
+// strided loops, three passes over the row.
 template <typename T, RowOp OP>
 __global__ __launch_bounds__(kBlock) void row_kernel_looped(
     const T* __restrict__ x, T* __restrict__ y, const void* __restrict__ gamma,
@@ -224,6 +366,38 @@ int dispatch_vec(const mfx_norm_args& a, hipStream_t s, int64_t nvec) {
   return launch_rows<T, PT, 256, 16, OP>(a, s);
 }
 
+template <typename T, typename PT, int LANES, int NV, RowOp OP>
+int launch_any(const mfx_norm_args& a, hipStream_t s) {
+  constexpr int block = LANES > kBlock ? LANES : kBlock, rpb = block / LANES;
+  hipLaunchKernelGGL((row_kernel_any<T, PT, LANES, NV, OP>), dim3((unsigned)((a.rows + rpb - 1) / rpb)), dim3(block), 0,
+                     s, static_cast<const T*>(a.x), static_cast<T*>(a.y), static_cast<const PT*>(a.gamma),
+                     static_cast<const PT*>(a.beta), a.rows, (int)a.n, a.x_row_stride, a.y_row_stride, a.eps);
+  return launch_status("row_kernel_any");
+}
+
+// Elements of a row that 1024 threads hold: 64 a thread, or 32 for the norms
+// (their parameters and second pass spill beside 64).
+template <RowOp OP>
+constexpr int64_t kAnyMax = is_softmax(OP) ? 65536 : 32768;
+
+// The fewest lanes whose registers hold the row.
+template <typename T, typename PT, RowOp OP>
+int dispatch_any(const mfx_norm_args& a, hipStream_t s) {
+  constexpr int VEC = Vec16<T>::N;
+  const int64_t runs = (a.n + VEC - 1) / VEC;
+  if (runs <= 64) return launch_any<T, PT, 64, 1, OP>(a, s);
+  if (runs <= 128) return launch_any<T, PT, 64, 2, OP>(a, s);
+  if (runs <= 256) return launch_any<T, PT, 64, 4, OP>(a, s);
+  if (runs <= 512) return launch_any<T, PT, 256, 2, OP>(a, s);
+  if (runs <= 1024) return launch_any<T, PT, 256, 4, OP>(a, s);
+  if (runs <= 2048) return launch_any<T, PT, 256, 8, OP>(a, s);
+  if (runs <= 4096) return launch_any<T, PT, 1024, 4, OP>(a, s);
+  if constexpr (VEC * 8192 <= kAnyMax<OP>)
+    if (runs <= 8192) return launch_any<T, PT, 1024, 8, OP>(a, s);
+  if constexpr (VEC * 16384 <= kAnyMax<OP>) return launch_any<T, PT, 1024, 16, OP>(a, s);
+  return fail(MFX_E_INVALID, "row too long for row_kernel_any");  // (excluded by kAnyMax)
+}
+
 template <typename T, RowOp OP>
 int dispatch_typed(const mfx_norm_args& a, hipStream_t s) {
   constexpr int VEC = Vec16<T>::N;
@@ -246,6 +420,13 @@ int dispatch_typed(const mfx_norm_args& a, hipStream_t s) {
       else return dispatch_vec<T, bf16, OP>(a, s, nvec);
     }
     return dispatch_vec<T, float, OP>(a, s, nvec);
+  }
+  if (a.n <= kAnyMax<OP> && pvec) {
+    if (params && a.param_dtype != MFX_F32) {
+      if constexpr (kF16) return dispatch_any<T, _Float16, OP>(a, s);
+      else return dispatch_any<T, bf16, OP>(a, s);
+    }
+    return dispatch_any<T, float, OP>(a, s);
   }
   hipLaunchKernelGGL((row_kernel_looped<T, OP>), dim3((unsigned)a.rows), dim3(kBlock), 0, s,
                      static_cast<const T*>(a.x), static_cast<T*>(a.y), a.gamma, a.beta,

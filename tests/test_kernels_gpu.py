@@ -83,6 +83,38 @@ def test_layer_norm_strided_rows_and_constant_rows(cuda, nat, oracle):
 
 
 
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("n", [1, 3, 255, 257, 511, 1025, 2049, 4099, 8193, 16385, 32767, 32769, 65535, 65537])
+def test_rows_of_any_length_and_alignment(cuda, nat, oracle, dt, n):
+    """LayerNorm, RMSNorm, softmax and log-softmax on rows off 16 bytes, at the
+    edges of the lanes-per-row variants and past the register-resident ones:
+    contiguous odd rows, and a view one element in with padded rows.  f32 bar:
+    the norms'; sums of n terms add at most n * 2^-24 relative to their size,
+    split over at least 64 lanes."""
+    td = {"f32": cuda.float32, "bf16": cuda.bfloat16, "f16": cuda.float16}[dt]
+    rng = np.random.default_rng(n)
+    rows = 5
+    x = rng.standard_normal((rows, n)) * 2 + 0.5
+    flat = cuda.zeros(1 + rows * (n + 3), dtype=td, device="cuda")
+    view = flat[1:].view(rows, n + 3)[:, :n]
+    view.copy_(dev(cuda, x, td))
+    g, b = dev(cuda, 1 + 0.1 * rng.standard_normal(n), td), dev(cuda, 0.1 * rng.standard_normal(n), td)
+    for xd in (dev(cuda, x, td), view):
+        xh = host(xd)
+        out = cuda.full((1 + rows * (n + 2),), 7.0, dtype=td, device="cuda")
+        ov = out[1:].view(rows, n + 2)[:, :n]
+        for got, ref in ((nat.layer_norm(xd, g, b, out=ov), oracle.layer_norm(xh, host(g), host(b), 1e-5)),
+                         (nat.rms_norm(xd, g), oracle.rms_norm(xh, host(g), 1e-5)),
+                         (nat.softmax(xd), oracle.softmax(xh)), (nat.log_softmax(xd), oracle.log_softmax(xh))):
+            got = host(got)
+            if dt == "f32":
+                assert np.abs(got - ref).max() <= F32_NORM_TOL * max(1.0, np.abs(ref).max())
+            else:
+                assert np.abs(got - ref).max() <= BF16_REL_TOL * max(np.abs(ref).max(), 1e-3)
+        pad = out[1:].view(rows, n + 2)[:, n:]
+        assert bool((pad == 7).all()) and float(out[0]) == 7.0  # nothing written beside the rows
+
+
 # ------------------------------------------------------- LayerNorm backward
 # mfx_layer_norm_bwd against the fp64 oracle (reference closed form
 # src/jax_mlx/layer_norm.py:59-76).  f32: ||out - ref||_inf <= 1e-5 *
