@@ -684,6 +684,9 @@ __global__ __launch_bounds__(kNT, D == 128 && MASKT != 0 && MASKT != kAnyMask ? 
     to[1].load(mrow, k0 + 16 + half * 8, Tk, odd);
   };
   if constexpr (RUNS) mask_load(mk, 0);
+  // A row with no visible key has no softmax: its lse is not finite and its
+  // gradient NaN, so a wavefront with such a row skips no block.
+  const bool may_skip = __ballot(qi < Tq && !(lse > -INFINITY)) == 0;
 
   // One 32-key block (MT) of the tile in stage ST:
   //   S^T = K Q^T and dP^T = V dO^T, their MFMAs alternating, K and V row
@@ -700,7 +703,7 @@ __global__ __launch_bounds__(kNT, D == 128 && MASKT != 0 && MASKT != kAnyMask ? 
     if constexpr (RUNS) {
       const bool ragged = EDGE && k0 + 32 > Tk;
       if (odd || ragged) place_runs(mk, mrow, k0 + half * 8, Tk, odd, ragged);
-      off = runs_all_off(mk);  // every dS is zero
+      off = may_skip && runs_all_off(mk);  // every dS is zero
     }
     bf16x8 db[2];
     if (!off) {

@@ -929,6 +929,21 @@ def test_sdpa_bwd_query_varying_mask_runs(cuda, nat, oracle, dt, mdt, D, tq, tk,
     check_grads(grads, refs, "bf16")
 
 
+@pytest.mark.parametrize("rows", [1, 64])
+@pytest.mark.parametrize("dt", ["bf16", "f32"])
+def test_sdpa_bwd_rows_without_a_visible_key(cuda, nat, dt, rows):
+    """The gradient of a row whose mask is only -inf is NaN, alone among rows
+    of its wavefront or with all of them; other rows' dQ is not."""
+    T, D = 150, 64
+    td = {"bf16": cuda.bfloat16, "f32": cuda.float32}[dt]
+    q, k, v = make_qkv(cuda, 81, (1, 2, T, D), (1, 2, T, D), td)
+    m = cuda.zeros(1, 1, T, T, device="cuda")
+    m[:, :, :rows] = -np.inf
+    dq = host(nat.sdpa_bwd(q, k, v, cuda.ones_like(q), mask=m)[0])
+    assert np.isnan(dq[:, :, :rows]).all()
+    assert np.isfinite(dq[:, :, rows:]).all()
+
+
 def test_sdpa_bwd_odd_head_size_generic(cuda, nat, oracle):
     grads, refs = bwd_case(cuda, nat, oracle, 43, (1, 3, 50, 80), (1, 3, 70, 80), "bf16", causal=True,
                            vshape=(1, 3, 70, 48))
