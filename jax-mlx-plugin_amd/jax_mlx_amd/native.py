@@ -445,15 +445,17 @@ _SDPA_BWD_PACK = struct.Struct("9PN7q32qf3i2P4q").pack
 
 
 def _mask_fields(mask):
-    """(pointer, [B, H, Tq, Tk] strides, dtype code) of an additive mask of at
-    most 4 dims (broadcast dims, of size 1, get stride 0); nulls for None."""
+    """(pointer, [B, H, Tq, Tk] strides, dtype code) of an additive mask
+    (broadcast dims, of size 1, get stride 0); nulls for None."""
     if mask is None:
         return 0, (0, 0, 0, 0), 0
-    nd = mask.dim()
-    if nd > 4:
-        raise ValueError("mask must have at most 4 dims [B, H, Tq, Tk]")
-    strides = (0,) * (4 - nd) + tuple(0 if n == 1 else st for n, st in zip(mask.shape, mask.stride()))
-    return mask.data_ptr(), strides, dtype_code(mask.dtype)
+    strides = tuple([0 if n == 1 else st for n, st in zip(mask.shape, mask.stride())])
+    return mask.data_ptr(), ((0,) * (4 - len(strides)) + strides)[:4], dtype_code(mask.dtype)
+
+
+def _f32(x):
+    """x as a C float holds it (past the range: an infinity, which packing refuses to make)."""
+    return ctypes.c_float(x).value
 
 
 def sdpa_args(q, k, v, out, *, scale=None, causal=False, mask=None, layout="bhtd",
@@ -462,6 +464,8 @@ def sdpa_args(q, k, v, out, *, scale=None, causal=False, mask=None, layout="bhtd
     _, Hkv, Tk, _ = _dims(k, layout)
     if scale is None:
         scale = 1.0 / (D ** 0.5)
+    if mask is not None and mask.dim() > 4:
+        raise ValueError("mask must have at most 4 dims [B, H, Tq, Tk]")
     mp, ms, md = _mask_fields(mask)
     if lse is not None and (lse.dtype != _torch().float32 or lse.numel() != B * Hq * Tq or not lse.is_contiguous()):
         raise ValueError("lse must be a contiguous f32 tensor of B * Hq * Tq elements")
@@ -471,7 +475,7 @@ def sdpa_args(q, k, v, out, *, scale=None, causal=False, mask=None, layout="bhtd
         workspace.data_ptr() if workspace is not None else 0,
         workspace.numel() * workspace.element_size() if workspace is not None else 0,
         B, Hq, Hkv, Tq, Tk, D, v.shape[-1], *_strides4(q, layout), *_strides4(k, layout), *_strides4(v, layout),
-        *_strides4(out, layout), *ms, float(scale), float(q_rms_eps) if q_rms_eps is not None else -1.0,
+        *_strides4(out, layout), *ms, _f32(scale), _f32(q_rms_eps) if q_rms_eps is not None else -1.0,
         1 if causal else 0, dtype_code(q.dtype), md, 0, lse.data_ptr() if lse is not None else 0))
 
 
@@ -540,7 +544,7 @@ def sdpa_bwd_args(q, k, v, dout, dq, dk, dv, *, scale=None, causal=False, mask=N
         workspace.numel() * workspace.element_size() if workspace is not None else 0,
         B, Hq, Hkv, Tq, Tk, D, v.shape[-1], *_strides4(q, layout), *_strides4(k, layout), *_strides4(v, layout),
         *_strides4(dout, layout), *_strides4(dq, layout), *_strides4(dk, layout), *_strides4(dv, layout), *ms,
-        float(scale), 1 if causal else 0, dtype_code(q.dtype), md,
+        _f32(scale), 1 if causal else 0, dtype_code(q.dtype), md,
         fwd_out.data_ptr() if fwd_out is not None else 0, fwd_lse.data_ptr() if fwd_lse is not None else 0,
         *(_strides4(fwd_out, layout) if fwd_out is not None else (0, 0, 0, 0))))
 

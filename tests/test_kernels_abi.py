@@ -333,3 +333,18 @@ def test_tanh_formula_accuracy():
     ref = np.tanh(x.astype(np.float64))
     ulp = np.abs(y - ref) / np.spacing(np.maximum(np.abs(ref), 1e-38).astype(f32)).astype(np.float64)
     assert ulp.max() <= 2.5, ulp.max()
+
+
+def test_sdpa_arguments_hold_what_a_c_struct_takes(native):
+    """A scale past the fp32 range is an infinity, and the backward reads the
+    first four dims of a mask, in the argument structs the binding packs."""
+    import torch
+
+    q, m = torch.zeros(2, 3, 4, 8), torch.zeros(2, 1, 4, 4, 1)
+    a = native.sdpa_args(q, q, q, q, scale=1e39, mask=m[..., 0], q_rms_eps=1e-6)
+    assert a.scale == float("inf") and list(a.mask_strides) == [16, 0, 4, 1]
+    assert a.q_rms_eps == ctypes.c_float(1e-6).value
+    b = native.sdpa_bwd_args(q, q, q, q, q, q, q, scale=-1e39, mask=m)
+    assert b.scale == float("-inf") and list(b.mask_strides) == [16, 0, 4, 1]
+    with pytest.raises(ValueError):
+        native.sdpa_args(q, q, q, q, mask=m)
