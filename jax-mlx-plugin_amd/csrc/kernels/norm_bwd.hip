@@ -7,8 +7,9 @@
 //   dx   = inv * (dxh - mean(dxh) - xhat * mean(dxh * xhat))
 //   dgamma = sum_rows(dy * xhat),  dbeta = sum_rows(dy)
 //
-// Pass 1 (ln_bwd_rows): a row is owned by 16 / 64 lanes of a wavefront or by
-// a 256-thread workgroup, as in the forward kernel; 16- and 64-lane groups
+// Pass 1 (ln_bwd_rows; ln_bwd_rows_any for rows off 16 bytes or of more than
+// 4096 elements): a row is owned by 16 / 64 lanes of a wavefront or by a
+// 256-thread workgroup (up to 1024 threads), as in the forward kernel; 16- and 64-lane groups
 // take rows in pairs with both rows' loads in flight together.  x and dy are
 // read once into registers as 16-byte vectors; mean and variance are recomputed from x
 // (two passes over registers), dx is written once.  Each lane keeps running
@@ -231,7 +232,132 @@ __global__ __launch_bounds__(kBlock) void ln_bwd_rows(
   }
 }
 
-// Rows that are unaligned or longer than the register-resident variants: the
+// ln_bwd_rows for rows at any alignment and up to 16 Ki elements: a row is
+// owned by a wavefront (rows in pairs, as above) or by a workgroup of 256, 512
+// or 1024 threads, read once in runs of 16 bytes, with at most 16 elements a
+// thread.
+//
+// Bound by HBM.  Such rows took the looped kernel, which reads x three times
+// and dy twice, one element per load, and updates its partial sums in memory:
+// [65536, 4095] f32 took 3110 us and takes 761 (4.2 TB/s; 653 at 4096 columns),
+// bf16 2776 and 566; [32768, 8192] f32 3108 and 603 (5.3 TB/s), bf16 2757 and
+// 613; [40000, 310] f32 184 and 56; [64, 101] f32 19 and 17.  16-bit rows wait:
+// a workgroup has one row of loads in flight.
+template <typename T, typename PT, int LANES, int NV>
+__global__ __launch_bounds__(LANES > kBlock ? LANES : kBlock) void ln_bwd_rows_any(
+    const T* __restrict__ x, const T* __restrict__ dy, T* __restrict__ dx, const PT* __restrict__ gamma,
+    float* __restrict__ partial, int64_t rows, int n, int64_t xs, int64_t gs, int64_t dxs, float eps) {
+  constexpr int VEC = Vec16<T>::N;
+  constexpr int BLOCK = LANES > kBlock ? LANES : kBlock, RPB = BLOCK / LANES;
+  constexpr int W = LANES * NV * VEC;  // columns one row's threads cover (>= n)
+  __shared__ float lds[2 * (BLOCK / 64)];
+  __shared__ float fold[RPB > 1 ? RPB * W : 1];
+  const int lane = threadIdx.x % LANES, grp = threadIdx.x / LANES;
+  const float inv_n = 1.0f / (float)n;
+  auto col = [&](int i) { return (i * LANES + lane) * VEC; };
+
+  float gv[NV][VEC], ag[NV][VEC], ab[NV][VEC];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) gv[i][j] = 1.f, ag[i][j] = ab[i][j] = 0.f;
+    if (gamma) load_run<PT, VEC>(gamma, col(i), n, 1.f, gv[i]);
+  }
+  // An absent row reads as zeros (row 0's address, no element of it).
+  auto load_row = [&](int64_t row, bool valid, float (&xv)[NV][VEC], float (&g)[NV][VEC]) {
+    const int64_t r = valid ? row : 0;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      load_run<T, VEC>(x + r * xs, col(i), valid ? n : 0, 0.f, xv[i]);
+      load_run<T, VEC>(dy + r * gs, col(i), valid ? n : 0, 0.f, g[i]);
+    }
+  };
+  auto finish_row = [&](int64_t row, bool valid, float (&xv)[NV][VEC], float (&g)[NV][VEC]) {
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) s += xv[i][j];
+    const float mean = row_reduce<LANES, false>(s, lds) * inv_n;
+    float q = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) {
+        xv[i][j] = col(i) + j < n ? xv[i][j] - mean : 0.f;
+        q += xv[i][j] * xv[i][j];
+      }
+    const float inv = rsqrtf(row_reduce<LANES, false>(q, lds) * inv_n + eps);
+    float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) {
+        xv[i][j] *= inv;  // xhat
+        const float d = g[i][j] * gv[i][j];
+        s1 += d;
+        s2 += d * xv[i][j];
+        if (valid) {
+          ag[i][j] = fmaf(g[i][j], xv[i][j], ag[i][j]);
+          ab[i][j] += g[i][j];
+        }
+      }
+    row_reduce_sum2<LANES>(s1, s2, lds);
+    const float m1 = s1 * inv_n, m2 = s2 * inv_n;
+    if (!valid) return;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      float o[VEC];
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) o[j] = inv * (g[i][j] * gv[i][j] - m1 - xv[i][j] * m2);
+      store_run<T, VEC>(dx + row * dxs, col(i), n, o);
+    }
+  };
+  const int64_t stride = (int64_t)gridDim.x * RPB;
+  if constexpr (LANES <= 64) {
+    for (int64_t row = (int64_t)blockIdx.x * RPB + grp; row < rows; row += 2 * stride) {
+      float xa[NV][VEC], ga[NV][VEC], xb[NV][VEC], gb[NV][VEC];
+      load_row(row, true, xa, ga);
+      load_row(row + stride, row + stride < rows, xb, gb);
+      finish_row(row, true, xa, ga);
+      finish_row(row + stride, row + stride < rows, xb, gb);
+    }
+  } else {
+    for (int64_t row = blockIdx.x; row < rows; row += stride) {
+      float xv[NV][VEC], g[NV][VEC];
+      load_row(row, true, xv, g);
+      finish_row(row, true, xv, g);
+    }
+  }
+
+  if (!partial) return;
+  float* const dst[2] = {partial + (int64_t)blockIdx.x * 2 * n, partial + ((int64_t)blockIdx.x * 2 + 1) * n};
+#pragma unroll
+  for (int pass = 0; pass < 2; ++pass) {
+    const float(&acc)[NV][VEC] = pass == 0 ? ag : ab;
+    if constexpr (RPB == 1) {
+#pragma unroll
+      for (int i = 0; i < NV; ++i) store_run<float, VEC>(dst[pass], col(i), n, acc[i]);
+    } else {
+      // Folds the wavefronts' rows: fold[grp][column].
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) fold[grp * W + col(i) + j] = acc[i][j];
+      __syncthreads();
+      for (int c = threadIdx.x; c < n; c += BLOCK) {
+        float t = 0.f;
+#pragma unroll
+        for (int r = 0; r < RPB; ++r) t += fold[r * W + c];
+        dst[pass][c] = t;
+      }
+      __syncthreads();
+    }
+  }
+}
+
+// Rows longer than the register-resident variants (and parameters of a type
+// those do not take): the
 // workgroup walks rows blockIdx.x, blockIdx.x + G, ...; thread t owns columns
 // t, t + 256, ... of the block's partial rows, which it updates in place
 // (no other thread touches them).
@@ -313,7 +439,8 @@ __global__ __launch_bounds__(64 * kParamWaves) void ln_bwd_params(
 }
 
 struct BwdPlan {
-  bool vector = false;
+  bool vector = false;  // ln_bwd_rows, or (any) ln_bwd_rows_any
+  bool any = false;
   int lanes = 0, nv = 0;
   int64_t groups = 0;  // G: workgroups of pass 1 = partial row pairs
 };
@@ -323,33 +450,34 @@ int vec_of(int dt) { return dt == MFX_F32 ? 4 : 8; }
 BwdPlan plan_bwd(const mfx_norm_bwd_args& a) {
   BwdPlan p;
   const int VEC = vec_of(a.dtype);
-  const int es = a.dtype == MFX_F32 ? 4 : 2;
   const int pbytes = a.param_dtype == MFX_F32 ? 4 : 2;
   const int palign = VEC * pbytes > 16 ? 16 : VEC * pbytes;
+  // The kernels that hold a row in registers read gamma stored as f32 or as
+  // bf16 (f16 rows: f32 or f16).
+  const bool ptype = !a.gamma || a.param_dtype == MFX_F32 ||
+                     a.param_dtype == (a.dtype == MFX_F16 ? MFX_F16 : MFX_BF16);
   const bool aligned = a.n % VEC == 0 && a.x_row_stride % VEC == 0 && a.dy_row_stride % VEC == 0 &&
                        a.dx_row_stride % VEC == 0 && (uintptr_t)a.x % 16 == 0 &&
                        (uintptr_t)a.dy % 16 == 0 && (uintptr_t)a.dx % 16 == 0 &&
-                       (!a.gamma || (uintptr_t)a.gamma % palign == 0) &&
-                       // Vector kernels read gamma stored as f32 or as bf16
-                       // (f16 rows: f32 or f16).
-                       (!a.gamma || a.param_dtype == MFX_F32 ||
-                        a.param_dtype == (a.dtype == MFX_F16 ? MFX_F16 : MFX_BF16));
-  const int64_t nvec = a.n / VEC;
-  (void)es;
+                       (!a.gamma || (uintptr_t)a.gamma % palign == 0);
+  const int64_t nvec = (a.n + VEC - 1) / VEC;
   // Register budget: at most 16 fp32 values per lane per row array.
   const int maxnv = 16 / VEC;
-  static const int kLanes[3] = {16, 64, 256};
-  if (aligned) {
-    for (int li = 0; li < 3 && !p.vector; ++li)
-      for (int nv = 1; nv <= maxnv; nv *= 2)
-        if (nvec <= (int64_t)kLanes[li] * nv) {
-          p.vector = true;
-          p.lanes = kLanes[li];
-          p.nv = nv;
-          break;
-        }
+  // Aligned rows of up to 256 lanes run ln_bwd_rows; ln_bwd_rows_any starts
+  // at a wavefront per row.
+  static const int kLanes[5] = {16, 64, 256, 512, 1024};
+  for (int li = 0; li < 5 && !p.vector && ptype; ++li) {
+    p.any = !aligned || li >= 3;
+    if (p.any && li == 0) continue;
+    for (int nv = li >= 3 ? maxnv : 1; nv <= maxnv; nv *= 2)
+      if (nvec <= (int64_t)kLanes[li] * nv) {
+        p.vector = true;
+        p.lanes = kLanes[li];
+        p.nv = nv;
+        break;
+      }
   }
-  const int64_t rpb = p.vector ? kBlock / p.lanes : 1;
+  const int64_t rpb = p.vector && p.lanes < kBlock ? kBlock / p.lanes : 1;
   // At least two rows per group, at most kMaxPartials partial row pairs.
   int64_t g = (a.rows + 2 * rpb - 1) / (2 * rpb);
   p.groups = g < 1 ? 1 : (g > kMaxPartials ? kMaxPartials : g);
@@ -364,9 +492,32 @@ void launch_rows_bwd(const mfx_norm_bwd_args& a, const BwdPlan& p, float* partia
                      a.eps);
 }
 
+template <typename T, typename PT, int LANES, int NV>
+void launch_any_bwd(const mfx_norm_bwd_args& a, const BwdPlan& p, float* partial, hipStream_t s) {
+  hipLaunchKernelGGL((ln_bwd_rows_any<T, PT, LANES, NV>), dim3((unsigned)p.groups),
+                     dim3(LANES > kBlock ? LANES : kBlock), 0, s, static_cast<const T*>(a.x),
+                     static_cast<const T*>(a.dy), static_cast<T*>(a.dx), static_cast<const PT*>(a.gamma), partial,
+                     a.rows, (int)a.n, a.x_row_stride, a.dy_row_stride, a.dx_row_stride, a.eps);
+}
+
+template <typename T, typename PT>
+void dispatch_any_bwd(const mfx_norm_bwd_args& a, const BwdPlan& p, float* partial, hipStream_t s) {
+  constexpr int MAX = 16 / Vec16<T>::N;
+  if (p.lanes == 1024) return launch_any_bwd<T, PT, 1024, MAX>(a, p, partial, s);
+  if (p.lanes == 512) return launch_any_bwd<T, PT, 512, MAX>(a, p, partial, s);
+  if (p.lanes == 256) {
+    if (p.nv == MAX) return launch_any_bwd<T, PT, 256, MAX>(a, p, partial, s);
+    return launch_any_bwd<T, PT, 256, MAX / 2>(a, p, partial, s);
+  }
+  if (p.nv == 1) return launch_any_bwd<T, PT, 64, 1>(a, p, partial, s);
+  if (p.nv == 2) return launch_any_bwd<T, PT, 64, 2>(a, p, partial, s);
+  return launch_any_bwd<T, PT, 64, MAX>(a, p, partial, s);
+}
+
 template <typename T, typename PT>
 void dispatch_rows_bwd(const mfx_norm_bwd_args& a, const BwdPlan& p, float* partial, hipStream_t s) {
   constexpr int VEC = Vec16<T>::N;
+  if (p.any) return dispatch_any_bwd<T, PT>(a, p, partial, s);
 #define MFX_LN_BWD_CASE(L, N)                                             \
   if (p.lanes == L && p.nv == N) {                                        \
     if constexpr (N * VEC <= 16) return launch_rows_bwd<T, PT, L, N>(a, p, partial, s); \

@@ -132,6 +132,60 @@ __device__ __forceinline__ void load_params(const void* p, int e, float* out) {
   }
 }
 
+// Runs of VEC elements from e on, of a row of n at any alignment: 16 bytes at
+// a time (a dword-aligned 16-byte load costs what an aligned one does), the
+// row's last, partial run element by element.
+template <typename T, int VEC>
+__device__ __forceinline__ void load_run(const T* row, int e, int n, float fill, float (&out)[VEC]) {
+  if (e + VEC <= n) {
+    if constexpr (sizeof(T) == 4) {
+      typedef float run_t __attribute__((ext_vector_type(4), aligned(4)));
+#pragma unroll
+      for (int c = 0; c < VEC / 4; ++c) {
+        const run_t r = *reinterpret_cast<const run_t*>(row + e + c * 4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) out[c * 4 + j] = r[j];
+      }
+    } else {
+      typedef uint32_t run_t __attribute__((ext_vector_type(VEC / 2), aligned(2)));
+      const run_t r = *reinterpret_cast<const run_t*>(row + e);
+#pragma unroll
+      for (int j = 0; j < VEC / 2; ++j) {
+        if constexpr (std::is_same<T, _Float16>::value) {
+          out[2 * j] = f16_lo(r[j]);
+          out[2 * j + 1] = f16_hi(r[j]);
+        } else {
+          out[2 * j] = __uint_as_float(r[j] << 16);
+          out[2 * j + 1] = __uint_as_float(r[j] & 0xffff0000u);
+        }
+      }
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) out[j] = e + j < n ? to_f32(row[e + j]) : fill;
+  }
+}
+
+template <typename T, int VEC>
+__device__ __forceinline__ void store_run(T* row, int e, int n, const float (&v)[VEC]) {
+  if (e + VEC <= n) {
+    if constexpr (sizeof(T) == 4) {
+      typedef float run_t __attribute__((ext_vector_type(4), aligned(4)));
+#pragma unroll
+      for (int c = 0; c < VEC; c += 4)
+        *reinterpret_cast<run_t*>(row + e + c) = run_t{v[c], v[c + 1], v[c + 2], v[c + 3]};
+    } else {
+      typedef uint32_t run_t __attribute__((ext_vector_type(4), aligned(2)));
+      const typename Vec16<T>::type w = pack16<T>(v);
+      *reinterpret_cast<run_t*>(row + e) = run_t{w.x, w.y, w.z, w.w};
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < VEC; ++j)
+      if (e + j < n) row[e + j] = from_f32<T>(v[j]);
+  }
+}
+
 // Sum / max over the LANES threads that own a row.  For LANES > 64 the
 // partials of the wavefronts meet in LDS.
 template <int LANES, bool kMax>

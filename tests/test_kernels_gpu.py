@@ -181,6 +181,37 @@ def test_layer_norm_bwd_without_gamma_strided_and_empty(cuda, nat, oracle):
     assert np.array_equal(host(dg4), host(dg)) and np.array_equal(host(db4), host(db))
 
 
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("rows,n", [
+    (9, 1), (9, 3), (8, 255), (9, 257), (9, 511), (9, 513), (9, 1025), (9, 2049), (9, 4097), (9, 4104), (9, 8191),
+    (9, 8200), (9, 16383), (9, 16384), (9, 16385), (8300, 33), (2100, 1031)])
+def test_layer_norm_bwd_rows_of_any_length_and_alignment(cuda, nat, oracle, dt, rows, n):
+    """Rows off 16 bytes, at the edges of the threads-per-row variants and past
+    the longest, as a contiguous tensor and as views one element in; groups
+    that walk several rows.  Parameters of the rows' type.  f32 bars: the other
+    cases'; a parameter gradient sums `rows` terms, within rows * 2^-24 of
+    their absolute sum."""
+    td = {"f32": cuda.float32, "bf16": cuda.bfloat16, "f16": cuda.float16}[dt]
+    rng = np.random.default_rng(n)
+    x, dy = rng.standard_normal((rows, n)) * 2 + 0.5, rng.standard_normal((rows, n))
+    gam = dev(cuda, 1 + 0.1 * rng.standard_normal(n), td)
+
+    def off(a, pad):
+        v = cuda.zeros(1 + rows * (n + pad), dtype=td, device="cuda")[1:].view(rows, n + pad)[:, :n]
+        v.copy_(dev(cuda, a, td))
+        return v
+
+    for xd, gd in ((dev(cuda, x, td), dev(cuda, dy, td)), (off(x, 3), off(dy, 2))):
+        ref = oracle.layer_norm_bwd(host(xd), host(gam), host(gd), 1e-5)
+        outs = [host(t) for t in nat.layer_norm_bwd(xd, gd, gam, eps=1e-5)]
+        if dt == "f32":
+            for o, r, terms in zip(outs, ref, (1, rows, rows)):
+                assert np.abs(o - r).max() <= max(F32_NORM_TOL, terms * 2.0 ** -24) * max(1.0, np.abs(r).max())
+        else:
+            for o, r in zip(outs, ref):
+                assert np.abs(o - r).max() <= BF16_REL_TOL * max(np.abs(r).max(), 1e-3)
+
+
 @pytest.mark.parametrize("dtype,shape", [("f32", (2, 4, 128)), ("f32", (9, 4096)), ("f32", (3, 77)),
                                          ("bf16", (16, 32, 1, 128)), ("bf16", (5, 2048))])
 def test_rms_norm(cuda, nat, oracle, dtype, shape):
