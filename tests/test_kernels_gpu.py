@@ -794,6 +794,23 @@ def test_sdpa_query_varying_mask_runs(cuda, nat, oracle, dt, mdt, D, tq, tk, for
     check_sdpa(a, ref, "bf16")
 
 
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("D", [32, 96])
+@pytest.mark.parametrize("tq,tk", [(70, 7), (130, 199), (256, 1024)])
+def test_sdpa_query_varying_mask_keeps_fp32_probabilities(cuda, nat, oracle, dt, D, tq, tk):
+    """At head sizes 32 and 96 P enters PV as two 16-bit terms: beside the
+    output's own rounding (2-norm 2^-9.2 of it in bf16, 2^-12.2 in f16) its
+    error of 2^-17 (f16: 2^-22) is lost, where one term would add as much
+    again."""
+    td = {"bf16": cuda.bfloat16, "f16": cuda.float16}[dt]
+    q, k, v = make_qkv(cuda, 64, (2, 2, tq, D), (2, 1, tk, D), td)
+    m = dev(cuda, np.random.default_rng(65).standard_normal((1, 2, tq, tk)), td)
+    out = host(nat.sdpa(q, k, v, scale=D ** -0.5, mask=m))
+    ref = oracle.sdpa(host(q), host(k), host(v), D ** -0.5, mask=np.broadcast_to(host(m), (2, 2, tq, tk)).copy())
+    rounded = host(cuda.from_numpy(ref).to(td))
+    assert np.linalg.norm(out - ref) <= 1.05 * np.linalg.norm(rounded - ref)
+
+
 @pytest.mark.parametrize("D", [64, 128, 256])
 def test_sdpa_query_varying_mask_extremes(cuda, nat, oracle, D):
     """A row of only -inf is NaN and its neighbours are not; a row whose first
