@@ -26,7 +26,7 @@ namespace {
 using namespace rowvec;
 
 constexpr int kMaxPartials = 1024;
-constexpr int kParamWaves = 16;
+constexpr int kParamWaves = 16, kParamCols = 32;
 
 template <typename T, typename PT, int LANES, int NV>
 __global__ __launch_bounds__(kBlock) void ln_bwd_rows(
@@ -407,34 +407,37 @@ __global__ __launch_bounds__(kBlock) void ln_bwd_rows_looped(
   }
 }
 
-// dgamma[c] = sum_p partial[p][0][c], dbeta[c] = sum_p partial[p][1][c]:
-// 64 columns per workgroup, its 16 wavefronts split the partial rows.
+// dgamma[c] = sum_p partial[p][0][c] (blockIdx.y 0), dbeta[c] = sum_p
+// partial[p][1][c] (blockIdx.y 1): kParamCols columns per workgroup, its
+// half-wavefronts split the partial rows.
+//
+// Bound by reading the partials (33.5 MB at 1024 x 4096).  64 columns of both
+// sums per workgroup left three quarters of the CUs idle there (31 us):
+// the whole backward of [65536, 4096] f32 goes from 653 to 632 us, of
+// [8192, 1024] from 47 to 29 (bf16 39 to 21), of [2^20, 512] from 1306 to 1291.
 template <typename PT>
 __global__ __launch_bounds__(64 * kParamWaves) void ln_bwd_params(
     const float* __restrict__ partial, int G, int64_t n, PT* __restrict__ dgamma,
     PT* __restrict__ dbeta) {
-  __shared__ float red[2][kParamWaves][64];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int64_t c = (int64_t)blockIdx.x * 64 + lane;
-  float sg = 0.f, sb = 0.f;
+  constexpr int SPLIT = 64 * kParamWaves / kParamCols;
+  __shared__ float red[SPLIT][kParamCols];
+  PT* out = blockIdx.y ? dbeta : dgamma;
+  if (!out) return;
+  const int lane = threadIdx.x % kParamCols, w = threadIdx.x / kParamCols;
+  const int64_t c = (int64_t)blockIdx.x * kParamCols + lane;
+  float t = 0.f;
   if (c < n) {
-    for (int p = w; p < G; p += kParamWaves) {
-      sg += partial[(int64_t)p * 2 * n + c];
-      sb += partial[(int64_t)p * 2 * n + n + c];
-    }
+    const float* col = partial + blockIdx.y * n + c;
+#pragma unroll 8
+    for (int p = w; p < G; p += SPLIT) t += col[(int64_t)p * 2 * n];
   }
-  red[0][w][lane] = sg;
-  red[1][w][lane] = sb;
+  red[w][lane] = t;
   __syncthreads();
   if (w == 0 && c < n) {
-    float tg = 0.f, tb = 0.f;
+    float sum = 0.f;
 #pragma unroll
-    for (int i = 0; i < kParamWaves; ++i) {
-      tg += red[0][i][lane];
-      tb += red[1][i][lane];
-    }
-    if (dgamma) dgamma[c] = from_f32<PT>(tg);
-    if (dbeta) dbeta[c] = from_f32<PT>(tb);
+    for (int i = 0; i < SPLIT; ++i) sum += red[i][lane];
+    out[c] = from_f32<PT>(sum);
   }
 }
 
@@ -619,15 +622,15 @@ int mfx_layer_norm_bwd(const mfx_norm_bwd_args* args, void* stream) {
   }
   if (!a.dgamma && !a.dbeta) return MFX_OK;
   const int G = a.rows == 0 ? 0 : (int)p.groups;
-  const unsigned blocks = (unsigned)((a.n + 63) / 64);
+  const dim3 blocks((unsigned)((a.n + kParamCols - 1) / kParamCols), 2);
   if (a.param_dtype == MFX_F32)
-    hipLaunchKernelGGL((ln_bwd_params<float>), dim3(blocks), dim3(64 * kParamWaves), 0, s, partial, G, a.n,
+    hipLaunchKernelGGL((ln_bwd_params<float>), blocks, dim3(64 * kParamWaves), 0, s, partial, G, a.n,
                        static_cast<float*>(a.dgamma), static_cast<float*>(a.dbeta));
   else if (a.param_dtype == MFX_F16)
-    hipLaunchKernelGGL((ln_bwd_params<_Float16>), dim3(blocks), dim3(64 * kParamWaves), 0, s, partial, G, a.n,
+    hipLaunchKernelGGL((ln_bwd_params<_Float16>), blocks, dim3(64 * kParamWaves), 0, s, partial, G, a.n,
                        static_cast<_Float16*>(a.dgamma), static_cast<_Float16*>(a.dbeta));
   else
-    hipLaunchKernelGGL((ln_bwd_params<bf16>), dim3(blocks), dim3(64 * kParamWaves), 0, s, partial, G, a.n,
+    hipLaunchKernelGGL((ln_bwd_params<bf16>), blocks, dim3(64 * kParamWaves), 0, s, partial, G, a.n,
                        static_cast<bf16*>(a.dgamma), static_cast<bf16*>(a.dbeta));
   return launch_status("ln_bwd_params");
 }
