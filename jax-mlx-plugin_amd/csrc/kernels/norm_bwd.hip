@@ -97,7 +97,9 @@ __global__ __launch_bounds__(kBlock) void ln_bwd_rows(
         q += xv[i][j] * xv[i][j];
       }
     }
-    const float inv = rsqrtf(row_reduce<LANES, false>(q, lds) * inv_n + eps);
+    // (An absent row's variance is 0, and with eps = 0 its rsqrt infinite.)
+    const float var = row_reduce<LANES, false>(q, lds) * inv_n;
+    const float inv = valid ? rsqrtf(var + eps) : 0.f;
     float s1 = 0.f, s2 = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; ++i)

@@ -14,6 +14,7 @@ pytestmark = pytest.mark.gpu
 F32_NORM_TOL = 1e-5
 F32_SDPA_TOL = 1e-4
 BF16_REL_TOL = 2e-2
+F16_REL_TOL = 5e-3  # as in test_f16_gpu.py
 
 
 @pytest.fixture(scope="module")
@@ -210,6 +211,23 @@ def test_layer_norm_bwd_rows_of_any_length_and_alignment(cuda, nat, oracle, dt, 
         else:
             for o, r in zip(outs, ref):
                 assert np.abs(o - r).max() <= BF16_REL_TOL * max(np.abs(r).max(), 1e-3)
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("n", [64, 511, 512, 4096, 4097])
+@pytest.mark.parametrize("rows", [1, 3, 2049])
+def test_layer_norm_bwd_without_eps(cuda, nat, oracle, dt, n, rows):
+    """eps = 0 with row counts that leave a pair of rows without its second
+    (16 and 64 lanes a row), on aligned and unaligned rows.  Bars: the other
+    cases'."""
+    td = {"f32": cuda.float32, "bf16": cuda.bfloat16, "f16": cuda.float16}[dt]
+    rng = np.random.default_rng(n + rows)
+    x, dy = dev(cuda, rng.standard_normal((rows, n)) * 2 + 0.5, td), dev(cuda, rng.standard_normal((rows, n)), td)
+    gam = dev(cuda, 1 + 0.1 * rng.standard_normal(n), td)
+    ref = oracle.layer_norm_bwd(host(x), host(gam), host(dy), 0.0)
+    for o, r, terms in zip(nat.layer_norm_bwd(x, dy, gam, eps=0.0), ref, (1, rows, rows)):
+        bar = max(F32_NORM_TOL, terms * 2.0 ** -24) if dt == "f32" else BF16_REL_TOL if dt == "bf16" else F16_REL_TOL
+        assert np.abs(host(o) - r).max() <= bar * max(1.0, np.abs(r).max())
 
 
 @pytest.mark.parametrize("dtype,shape", [("f32", (2, 4, 128)), ("f32", (9, 4096)), ("f32", (3, 77)),
