@@ -109,6 +109,18 @@ __device__ __forceinline__ void col_product(const float* tile, const f32x16& w, 
     }
 }
 
+// Whether a lane's sums hold a NaN or an infinity.
+template <int D>
+__device__ __forceinline__ bool nonfinite(const f32x16 (&acc)[D / 32]) {
+  float t[4] = {};  // zeros or NaN
+#pragma unroll
+  for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) t[i & 3] = fmaf(acc[dt][i], 0.f, t[i & 3]);
+  const float any = (t[0] + t[1]) + (t[2] + t[3]);
+  return __ballot(any != any) != 0;
+}
+
 // The lane's half of row `row` as a B operand, zero when !valid.
 template <int D>
 __device__ __forceinline__ void load_row(const float* row, bool valid, int half, float (&r)[D / 2]) {
@@ -134,6 +146,95 @@ __device__ __forceinline__ void store_row(float* row, const f32x16 (&acc)[D / 32
       for (int e = 0; e < 4; ++e) w[e] = acc[dt][g * 4 + e] * mul;
       *reinterpret_cast<f32x4*>(row + dt * 32 + g * 8 + half * 4) = w;
     }
+}
+
+// A matrix product multiplies the rows that causality hides too, by zero,
+// which is NaN where such a row is not finite; but hidden rows must not take
+// part at all.  So where a causal call's sums are not all finite, the
+// wavefront's 32 output rows are computed again by these, one row at a time
+// from what it sees: a lane per row of the other axis for the scores, then per
+// feature for the sums.  (Asking the sums costs D / 2 instructions, D in dkdv,
+// once a wavefront: [16,8,20,64] goes from 14.9 to 15.3 us, [1,1,2048,64] stays
+// at 539.)
+//
+// Features f*64 + lane of a row.
+template <int D>
+constexpr int kFeat = (D + 63) / 64;
+
+template <int D>
+__device__ __forceinline__ float row_dot(const float* a, const float* b) {
+  float s = 0.f;
+#pragma unroll 4
+  for (int d = 0; d < D; ++d) s = fmaf(a[d], b[d], s);
+  return s;
+}
+
+template <int D, int MT>
+__device__ __forceinline__ float row_score(const SdpaBwdParams& p, const float* q, const float* k, int64_t moff) {
+  float s = row_dot<D>(q, k) * p.scale_log2;
+  if constexpr (MT != 0) s += mask_log2(load_mask_t<MT>(p.mask, moff));
+  return s;
+}
+
+template <int D>
+__device__ __forceinline__ void add_row(const float* row, float w, int lane, float (&acc)[kFeat<D>]) {
+#pragma unroll
+  for (int f = 0; f < kFeat<D>; ++f)
+    if (f * 64 + lane < D) acc[f] = fmaf(w, row[f * 64 + lane], acc[f]);
+}
+
+template <int D>
+__device__ __forceinline__ void put_row(float* row, float mul, int lane, const float (&acc)[kFeat<D>]) {
+#pragma unroll
+  for (int f = 0; f < kFeat<D>; ++f)
+    if (f * 64 + lane < D) row[f * 64 + lane] = acc[f] * mul;
+}
+
+// dQ of query i, which sees keys 0 .. i.
+template <int D, int MT>
+__device__ __forceinline__ void dq_row(const SdpaBwdParams& p, int b, int h, int i, float lse, float delta, int lane) {
+  const int hk = h / p.group;
+  const float* q = static_cast<const float*>(p.q) + b * p.qs[0] + h * p.qs[1] + (int64_t)i * p.qs[2];
+  const float* g = static_cast<const float*>(p.dout) + b * p.dos[0] + h * p.dos[1] + (int64_t)i * p.dos[2];
+  const float* k = static_cast<const float*>(p.k) + b * p.ks[0] + hk * p.ks[1];
+  const float* v = static_cast<const float*>(p.v) + b * p.vs[0] + hk * p.vs[1];
+  const int64_t mrow = MT ? b * p.ms[0] + h * p.ms[1] + (int64_t)i * p.ms[2] : 0;
+  float acc[kFeat<D>] = {};
+  const int end = min(p.Tk, i + 1);
+  for (int kb = 0; kb < end; kb += 64) {
+    const int j = min(kb + lane, end - 1);
+    const float x = row_score<D, MT>(p, q, k + (int64_t)j * p.ks[2], mrow + (MT ? j * p.ms[3] : 0));
+    const float ds = __builtin_amdgcn_exp2f(x - lse) * (row_dot<D>(g, v + (int64_t)j * p.vs[2]) - delta);
+    const int n = min(64, end - kb);
+    for (int jj = 0; jj < n; ++jj) add_row<D>(k + (int64_t)(kb + jj) * p.ks[2], __shfl(ds, jj, 64), lane, acc);
+  }
+  put_row<D>(static_cast<float*>(p.dq) + b * p.dqs[0] + h * p.dqs[1] + (int64_t)i * p.dqs[2], p.scale, lane, acc);
+}
+
+// dK and dV of key j, which queries j .. Tq - 1 of every head of the group see.
+template <int D, int MT>
+__device__ __forceinline__ void dkdv_row(const SdpaBwdParams& p, int b, int hk, int j, int lane) {
+  const float* k = static_cast<const float*>(p.k) + b * p.ks[0] + hk * p.ks[1] + (int64_t)j * p.ks[2];
+  const float* v = static_cast<const float*>(p.v) + b * p.vs[0] + hk * p.vs[1] + (int64_t)j * p.vs[2];
+  float dk[kFeat<D>] = {}, dv[kFeat<D>] = {};
+  for (int h = hk * p.group; h < (hk + 1) * p.group; ++h) {
+    const float* q = static_cast<const float*>(p.q) + b * p.qs[0] + h * p.qs[1];
+    const float* g = static_cast<const float*>(p.dout) + b * p.dos[0] + h * p.dos[1];
+    const int64_t mcol = MT ? b * p.ms[0] + h * p.ms[1] + j * p.ms[3] : 0, rows = ((int64_t)b * p.Hq + h) * p.Tq;
+    for (int qb = j; qb < p.Tq; qb += 64) {
+      const int i = min(qb + lane, p.Tq - 1);
+      const float x = row_score<D, MT>(p, q + (int64_t)i * p.qs[2], k, mcol + (MT ? i * p.ms[2] : 0));
+      const float pr = __builtin_amdgcn_exp2f(x - p.lse[rows + i]);
+      const float ds = pr * (row_dot<D>(g + (int64_t)i * p.dos[2], v) - p.delta[rows + i]);
+      const int n = min(64, p.Tq - qb);
+      for (int ii = 0; ii < n; ++ii) {
+        add_row<D>(q + (int64_t)(qb + ii) * p.qs[2], __shfl(ds, ii, 64), lane, dk);
+        add_row<D>(g + (int64_t)(qb + ii) * p.dos[2], __shfl(pr, ii, 64), lane, dv);
+      }
+    }
+  }
+  put_row<D>(static_cast<float*>(p.dk) + b * p.dks[0] + hk * p.dks[1] + (int64_t)j * p.dks[2], p.scale, lane, dk);
+  put_row<D>(static_cast<float*>(p.dv) + b * p.dvs[0] + hk * p.dvs[1] + (int64_t)j * p.dvs[2], 1.f, lane, dv);
 }
 
 // (head, block) of a workgroup: a head's blocks on one XCD (workgroups are
@@ -233,6 +334,11 @@ __global__ __launch_bounds__(64 * NW, D <= 64 ? 2 : 1) void bwd_f32_dq_kernel(Sd
     if (t + 1 < ntiles) ld.store(k_lds[(t + 1) & 1], v_lds[(t + 1) & 1], tid);
     __syncthreads();
   }
+  if (causal && __builtin_expect(nonfinite<D>(dq), false)) {
+    for (int r = 0; r < 32 && q0 + r < Tq; ++r)
+      dq_row<D, MT>(p, b, h, q0 + r, __shfl(lse, r, 64), __shfl(delta, r, 64), lane);
+    return;
+  }
   if (qv)
     store_row<D>(static_cast<float*>(p.dq) + b * p.dqs[0] + h * p.dqs[1] + (int64_t)qi * p.dqs[2], dq, half, p.scale);
 }
@@ -326,6 +432,10 @@ __global__ __launch_bounds__(64 * NW, D <= 64 ? 2 : 1) void bwd_f32_dkdv_kernel(
     }
     if (it + 1 < n) store((it + 1) & 1);
     __syncthreads();
+  }
+  if (causal && __builtin_expect(nonfinite<D>(dk) || nonfinite<D>(dv), false)) {
+    for (int r = 0; r < 32 && k0 + r < Tk; ++r) dkdv_row<D, MT>(p, b, hk, k0 + r, lane);
+    return;
   }
   if (key < Tk) {
     store_row<D>(static_cast<float*>(p.dk) + b * p.dks[0] + hk * p.dks[1] + (int64_t)key * p.dks[2], dk, half, p.scale);

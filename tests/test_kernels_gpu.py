@@ -1049,6 +1049,46 @@ def test_sdpa_bwd_f32_matrix_cores(cuda, nat, oracle, D, B, hq, hkv, tq, tk, cau
     check_grads(grads, refs, "f32")
 
 
+@pytest.mark.parametrize("D", [32, 64, 96, 128])
+@pytest.mark.parametrize("B,hq,hkv,tq,tk,mdt", [
+    (1, 4, 2, 70, 70, None), (2, 2, 2, 70, 100, "f32"), (1, 2, 1, 64, 33, "bf16"),
+    (16, 32, 32, 70, 70, None),  # four wavefronts per workgroup
+])
+@pytest.mark.parametrize("which,rows,value", [
+    ("k", (40,), np.nan), ("k", (29, 31), -np.inf), ("q", (37,), np.nan), ("q", (63,), np.inf),
+    ("g", (50,), np.inf), ("g", (33, 35), np.nan), ("k", (75,), np.nan)])
+def test_sdpa_bwd_f32_hidden_rows_that_are_not_finite(cuda, nat, D, B, hq, hkv, tq, tk, mdt, which, rows, value):
+    """A NaN or an infinity in a row that causality hides from a query (or
+    key) does not reach its gradient, also from the same tile, and reaches
+    those that see it as on the per-row kernels (the same call with rows off
+    16 bytes).  Finite values: the other f32 cases' bar."""
+    g = cuda.Generator(device="cuda").manual_seed(D + tk)
+    q, k, v, go = (cuda.randn(B, h, t, D, generator=g, device="cuda")
+                   for h, t in ((hq, tq), (hkv, tk), (hkv, tk), (hq, tq)))
+    mask = None
+    if mdt:
+        mask = cuda.randn(B, 1, tq, tk, generator=g, device="cuda").to({"f32": cuda.float32, "bf16": cuda.bfloat16}[mdt])
+    rows = [r for r in rows if r < (tk if which == "k" else tq)]
+    lse = cuda.empty(B * hq * tq, device="cuda")
+    for r in rows:
+        {"q": q, "k": k, "g": go}[which][:, -1, r, ::5] = value
+    out = nat.sdpa(q, k, v, causal=True, mask=mask, lse=lse)
+    wide = cuda.zeros(B, hkv, tk, D + 1, device="cuda")
+    wide[..., :D] = k
+    kw = dict(causal=True, mask=mask, fwd_out=out, fwd_lse=lse)
+    got, want = nat.sdpa_bwd(q, k, v, go, **kw), nat.sdpa_bwd(q, wide[..., :D], v, go, **kw)
+    for name, a, b in zip(("dq", "dk", "dv"), got, want):
+        a, b = host(a), host(b)
+        assert np.array_equal(np.isfinite(a), np.isfinite(b)), name
+        odd = ~np.isfinite(b)
+        assert np.array_equal(a[odd], b[odd], equal_nan=True), name
+        assert np.abs(a[~odd] - b[~odd]).max(initial=0) <= F32_SDPA_TOL * np.abs(b[~odd]).max(initial=1), name
+    if rows and which == "k":
+        assert bool(cuda.isfinite(got[0][:, :, :min(rows)]).all())
+    if rows and which == "g":
+        assert bool(cuda.isfinite(got[2][:, :, max(rows) + 1:]).all())
+
+
 def test_sdpa_bwd_f32_unaligned_rows(cuda, nat, oracle):
     """Row strides off 16 bytes and overlapping rows stay on the per-row
     kernels, with the same gradients."""
