@@ -303,10 +303,10 @@ int mfx_sdpa_bwd(const mfx_sdpa_bwd_args* args, void* stream);
 size_t mfx_sdpa_bwd_workspace_size(const mfx_sdpa_bwd_args* args);
 
 /* Which backward kernels mfx_sdpa_bwd would launch: "mfma_bf16_d128",
- * "mfma_bf16_d96" (through the padded copies), ... for the 16-bit
- * matrix-core kernels; "generic" for every other call, which are the per-row
- * kernels and, for f32 at head sizes 32, 64, 96 and 128 with 16-byte aligned
- * rows, the fp32 matrix-core kernels.  NULL if the arguments are invalid. */
+ * "mfma_bf16_d96" (through the padded copies), "mfma_f32_d64", ... for the
+ * matrix-core kernels (f32: head sizes 32, 64, 96 and 128 with 16-byte
+ * aligned rows that do not overlap); "generic" for the per-row kernels, which
+ * take every other call.  NULL if the arguments are invalid. */
 const char* mfx_sdpa_bwd_kernel_name(const mfx_sdpa_bwd_args* args);
 
 /* ==========================================================================

@@ -407,7 +407,10 @@ const char* mfx_sdpa_bwd_kernel_name(const mfx_sdpa_bwd_args* args) {
     static const char* const padded[2][2] = {{"mfma_bf16_d32", "mfma_bf16_d96"}, {"mfma_f16_d32", "mfma_f16_d96"}};
     return padded[pl.p.dtype == MFX_F16][pl.p.D == 96];
   }
-  // f32 calls keep the one name on either of their routes.
+  if (pl.f32) {
+    static const char* const f32[4] = {"mfma_f32_d32", "mfma_f32_d64", "mfma_f32_d96", "mfma_f32_d128"};
+    return f32[pl.p.D / 32 - 1];
+  }
   if (!pl.mfma) return "generic";
   if (pl.p.dtype == MFX_F16) return pl.p.D == 128 ? "mfma_f16_d128" : "mfma_f16_d64";
   return pl.p.D == 128 ? "mfma_bf16_d128" : "mfma_bf16_d64";

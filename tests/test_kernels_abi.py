@@ -117,6 +117,31 @@ def test_short_kv_row_strides_leave_buffer_resource_kernels(native):
         assert lib.mfx_sdpa_bwd_kernel_name(ctypes.byref(a)).decode() == "generic", which
 
 
+def test_f32_backward_route_is_named(native):
+    """f32 calls at head sizes 32 to 128 take the fp32 matrix-core kernels and
+    say so; rows off 16 bytes, overlapping rows, other head sizes and Dv != D
+    take the per-row ones."""
+    import ctypes
+
+    import torch
+
+    name = lambda a: native.load().mfx_sdpa_bwd_kernel_name(ctypes.byref(a)).decode()
+    for D in (32, 64, 96, 128):
+        q, k = (torch.zeros(1, h, t, D) for h, t in ((4, 50), (2, 70)))
+        assert native.sdpa_bwd_kernel_name(q, k, k) == f"mfma_f32_d{D}"
+        assert native.sdpa_bwd_kernel_name(q, torch.zeros(1, 2, 70, D + 1)[..., :D], k) == "generic"
+        assert native.sdpa_bwd_kernel_name(q, k, k[:, :, :1].expand(1, 2, 70, D)) == "generic"
+        assert native.sdpa_bwd_kernel_name(torch.zeros(4 * 50 * D + 1)[1:].view(1, 4, 50, D), k, k) == "generic"
+        a = native.sdpa_bwd_args(q, k, k, q, q, k, k)
+        a.dk_strides[1] += 2
+        assert name(a) == "generic"
+    q, k = torch.zeros(1, 2, 50, 80), torch.zeros(1, 2, 50, 80)
+    assert native.sdpa_bwd_kernel_name(q, k, k) == "generic"
+    q, k, v = torch.zeros(1, 2, 50, 64), torch.zeros(1, 2, 50, 64), torch.zeros(1, 2, 50, 32)
+    a = native.sdpa_bwd_args(q, k, v, v, q, k, v)
+    assert name(a) == "generic"
+
+
 def test_decode_workspace_is_sized(native):
     import torch
 

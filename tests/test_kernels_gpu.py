@@ -1034,6 +1034,8 @@ def test_sdpa_bwd_f32_matrix_cores(cuda, nat, oracle, D, B, hq, hkv, tq, tk, cau
         m = np.random.default_rng(D).standard_normal((B, 1, tq, tk)).astype(np.float32)
         m[:, :, :, 3] = -np.inf
         mask = dev(cuda, m, {"f32": cuda.float32, "bf16": cuda.bfloat16, "f16": cuda.float16}[mdt])
+    td = cuda.empty(shape(hq, tq), device="cuda"), cuda.empty(shape(hkv, tk), device="cuda")
+    assert nat.sdpa_bwd_kernel_name(td[0], td[1], td[1], causal=causal, mask=mask, layout=layout) == f"mfma_f32_d{D}"
     if B == 16:  # one batch's heads against the oracle, the others against a call of their own
         g = cuda.Generator(device="cuda").manual_seed(D)
         q, k, v, go = (cuda.randn(shape(h, t), generator=g, device="cuda")
@@ -1075,6 +1077,8 @@ def test_sdpa_bwd_f32_hidden_rows_that_are_not_finite(cuda, nat, D, B, hq, hkv, 
     out = nat.sdpa(q, k, v, causal=True, mask=mask, lse=lse)
     wide = cuda.zeros(B, hkv, tk, D + 1, device="cuda")
     wide[..., :D] = k
+    assert nat.sdpa_bwd_kernel_name(q, k, v, causal=True, mask=mask) == f"mfma_f32_d{D}"
+    assert nat.sdpa_bwd_kernel_name(q, wide[..., :D], v, causal=True, mask=mask) == "generic"
     kw = dict(causal=True, mask=mask, fwd_out=out, fwd_lse=lse)
     got, want = nat.sdpa_bwd(q, k, v, go, **kw), nat.sdpa_bwd(q, wide[..., :D], v, go, **kw)
     for name, a, b in zip(("dq", "dk", "dv"), got, want):
@@ -1100,9 +1104,11 @@ def test_sdpa_bwd_f32_unaligned_rows(cuda, nat, oracle):
     wide = cuda.zeros(B, H, T, D + 1, device="cuda")
     wide[..., :D] = k
     refs = nat.sdpa_bwd(q, k, v, g)
+    assert nat.sdpa_bwd_kernel_name(q, wide[..., :D], v) == "generic"
     for a, r in zip(nat.sdpa_bwd(q, wide[..., :D], v, g), refs):
         assert np.abs(host(a) - host(r)).max() <= F32_SDPA_TOL * max(1.0, np.abs(host(r)).max())
     v1 = v[:, :, :1].expand(B, H, T, D)
+    assert nat.sdpa_bwd_kernel_name(q, k, v1) == "generic"
     dense = nat.sdpa_bwd(q, k, v1.contiguous(), g)
     dq, dk, dv = cuda.empty_like(q), cuda.empty_like(k), cuda.empty_like(v)
     a = nat.sdpa_bwd_args(q, k, v1, g, dq, dk, dv)
@@ -1134,7 +1140,10 @@ def test_sdpa_bwd_kernel_selection(cuda, nat):
     assert nat.sdpa_bwd_kernel_name(q, k, v) == "mfma_bf16_d128"
     q, k, v = make_qkv(cuda, 1, (1, 2, 64, 64), (1, 2, 64, 64), cuda.bfloat16)
     assert nat.sdpa_bwd_kernel_name(q, k, v, causal=True) == "mfma_bf16_d64"
-    q, k, v = make_qkv(cuda, 1, (1, 2, 64, 64), (1, 2, 64, 64), cuda.float32)
+    for D in (32, 64, 96, 128):
+        q, k, v = make_qkv(cuda, 1, (1, 2, 64, D), (1, 2, 64, D), cuda.float32)
+        assert nat.sdpa_bwd_kernel_name(q, k, v) == f"mfma_f32_d{D}"
+    q, k, v = make_qkv(cuda, 1, (1, 2, 64, 80), (1, 2, 64, 80), cuda.float32)
     assert nat.sdpa_bwd_kernel_name(q, k, v) == "generic"
 
 
