@@ -259,7 +259,9 @@ const char* mfx_sdpa_kernel_name(const mfx_sdpa_args* args);
  * custom_call @mlx_sdpa_bwd interface (q, k, v, grad_out) has no slot for
  * them, and its mx::vjp recomputes.  Workspace:
  * mfx_sdpa_bwd_workspace_size() bytes, or NULL for library scratch.
- * Deterministic: no atomics.
+ * Deterministic: no atomics.  dq, dk and dv must not share memory with the
+ * inputs or each other; only f32 calls may store dq over q or dout, row by row
+ * (on the per-row kernels, a slower route).
  * Replaces mx::vjp of fast::scaled_dot_product_attention behind custom_call
  * @mlx_sdpa_bwd (reference src/jax_mlx_pjrt.cpp:8151-8206; closed form
  * src/jax_mlx/sdpa.py:65-87).
@@ -305,7 +307,7 @@ size_t mfx_sdpa_bwd_workspace_size(const mfx_sdpa_bwd_args* args);
 /* Which backward kernels mfx_sdpa_bwd would launch: "mfma_bf16_d128",
  * "mfma_bf16_d96" (through the padded copies), "mfma_f32_d64", ... for the
  * matrix-core kernels (f32: head sizes 32, 64, 96 and 128 with 16-byte
- * aligned rows that do not overlap); "generic" for the per-row kernels, which
+ * aligned rows that do not overlap, and dq apart from q and dout); "generic" for the per-row kernels, which
  * take every other call.  NULL if the arguments are invalid. */
 const char* mfx_sdpa_bwd_kernel_name(const mfx_sdpa_bwd_args* args);
 

@@ -210,6 +210,26 @@ __global__ __launch_bounds__(256) void pad_rows_kernel(const uint16_t* __restric
   }
 }
 
+// Bytes [first, last] of a [B, H, T, D] tensor (feature stride 1).
+struct Span {
+  intptr_t first, last;
+};
+Span span(const void* ptr, const int64_t* st, int64_t B, int64_t H, int64_t T, int64_t D, int64_t size) {
+  Span r{0, D - 1};
+  const int64_t n[3] = {B, H, T};
+  for (int i = 0; i < 3; ++i) (st[i] < 0 ? r.first : r.last) += (n[i] - 1) * st[i];
+  return {(intptr_t)ptr + r.first * size, (intptr_t)ptr + (r.last + 1) * size - 1};
+}
+
+// Whether dQ shares bytes with q or dO.
+bool dq_in_place(const SdpaBwdParams& p) {
+  const int64_t es = dtype_size(p.dtype);
+  const Span d = span(p.dq, p.dqs, p.B, p.Hq, p.Tq, p.D, es);
+  for (const Span& s : {span(p.q, p.qs, p.B, p.Hq, p.Tq, p.D, es), span(p.dout, p.dos, p.B, p.Hq, p.Tq, p.Dv, es)})
+    if (d.first <= s.last && s.first <= d.last) return true;
+  return false;
+}
+
 struct BwdPlan {
   SdpaBwdParams p{};
   SdpaParams fwd{};
@@ -329,7 +349,9 @@ int make_bwd_plan(const mfx_sdpa_bwd_args* a, BwdPlan& out) {
   f.num_splits = 1;
   f.split_len = p.Tk;
   out.mfma = bwd_mfma_supports(p);
-  out.f32 = bwd_f32_supports(p);
+  // The matrix-core kernels write dQ before dK / dV read q and dO; the per-row
+  // ones read a row of q and dO last for the dQ row that may take its place.
+  out.f32 = bwd_f32_supports(p) && !dq_in_place(p);
   // The copies move 16-byte chunks: every tensor 16-byte aligned with
   // strides of whole chunks (the recomputed O is the workspace's).
   auto chunked = [&]() {

@@ -565,8 +565,10 @@ def sdpa_bwd(q, k, v, dout, *, scale=None, causal=False, mask=None, layout="bhtd
 
 
 def sdpa_bwd_kernel_name(q, k, v, **kw) -> str:
-    """Which backward kernels mfx_sdpa_bwd picks (host-only query)."""
+    """Which backward kernels mfx_sdpa_bwd picks (host-only query) for outputs
+    of their own."""
     a = sdpa_bwd_args(q, k, v, q, q, k, v, **kw)
+    a.dq = a.dk = a.dv = 256  # (apart from the inputs, 16-byte aligned)
     name = load().mfx_sdpa_bwd_kernel_name(ctypes.byref(a))
     if name is None:
         raise MfxError(-1, load().mfx_last_error().decode())

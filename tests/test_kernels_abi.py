@@ -132,9 +132,19 @@ def test_f32_backward_route_is_named(native):
         assert native.sdpa_bwd_kernel_name(q, torch.zeros(1, 2, 70, D + 1)[..., :D], k) == "generic"
         assert native.sdpa_bwd_kernel_name(q, k, k[:, :, :1].expand(1, 2, 70, D)) == "generic"
         assert native.sdpa_bwd_kernel_name(torch.zeros(4 * 50 * D + 1)[1:].view(1, 4, 50, D), k, k) == "generic"
-        a = native.sdpa_bwd_args(q, k, k, q, q, k, k)
+        a = native.sdpa_bwd_args(q, k, k, q, q.clone(), k, k)
+        assert name(a) == f"mfma_f32_d{D}"
         a.dk_strides[1] += 2
         assert name(a) == "generic"
+    # dq over q or dO, wholly or in part; beside them in one buffer it is apart.
+    q, g, dq, k = (torch.zeros(1, 2, 50, 64) for _ in range(4))
+    for d, want in ((dq, "mfma_f32_d64"), (q, "generic"), (g, "generic")):
+        assert name(native.sdpa_bwd_args(q, k, k, g, d, dq.clone(), dq.clone())) == want
+    buf = torch.zeros(3 * q.numel())
+    rows = [buf[i * q.numel():(i + 1) * q.numel()].view(q.shape) for i in range(3)]
+    assert name(native.sdpa_bwd_args(rows[0], k, k, rows[2], rows[1], dq, dq)) == "mfma_f32_d64"
+    last = buf[q.numel() - 4:][:q.numel()].view(q.shape)
+    assert name(native.sdpa_bwd_args(rows[0], k, k, rows[2], last, dq, dq)) == "generic"
     q, k = torch.zeros(1, 2, 50, 80), torch.zeros(1, 2, 50, 80)
     assert native.sdpa_bwd_kernel_name(q, k, k) == "generic"
     q, k, v = torch.zeros(1, 2, 50, 64), torch.zeros(1, 2, 50, 64), torch.zeros(1, 2, 50, 32)

@@ -1117,6 +1117,29 @@ def test_sdpa_bwd_f32_unaligned_rows(cuda, nat, oracle):
         assert np.abs(host(o) - host(r)).max() <= F32_SDPA_TOL * max(1.0, np.abs(host(r)).max())
 
 
+@pytest.mark.parametrize("over", ["q", "g"])
+@pytest.mark.parametrize("saved", [False, True])
+@pytest.mark.parametrize("D,causal", [(32, False), (64, True), (96, True), (128, False)])
+def test_sdpa_bwd_f32_dq_in_place(cuda, nat, D, causal, saved, over):
+    """dq stored over q or dO row by row: the gradients of the call with
+    outputs of its own (the other f32 cases' bar)."""
+    import ctypes
+
+    gen = cuda.Generator(device="cuda").manual_seed(D)
+    q, k, v, g = (cuda.randn(2, h, t, D, generator=gen, device="cuda") for h, t in ((4, 70), (2, 90), (2, 90), (4, 70)))
+    lse = cuda.empty(2 * 4 * 70, device="cuda")
+    kw = dict(causal=causal)
+    if saved:
+        kw |= dict(fwd_out=nat.sdpa(q, k, v, causal=causal, lse=lse), fwd_lse=lse)
+    refs = nat.sdpa_bwd(q, k, v, g, **kw)
+    dq = {"q": q, "g": g}[over]
+    dk, dv = cuda.empty_like(k), cuda.empty_like(v)
+    a = nat.sdpa_bwd_args(q, k, v, g, dq, dk, dv, **kw)
+    nat.check(nat.load().mfx_sdpa_bwd(ctypes.byref(a), cuda.cuda.current_stream().cuda_stream))
+    for name, o, r in zip(("dq", "dk", "dv"), (dq, dk, dv), refs):
+        assert np.abs(host(o) - host(r)).max() <= F32_SDPA_TOL * max(1.0, np.abs(host(r)).max()), name
+
+
 def test_sdpa_bwd_known_answers(cuda, nat):
     """Tk = 1: out = v, so dv = sum over query rows of dO and dq = dk = 0.
     Identical keys: P is uniform 1/Tk, so dq = 0 and every dv_j is the sum of
