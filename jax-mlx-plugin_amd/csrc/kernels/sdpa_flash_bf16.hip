@@ -194,6 +194,26 @@ __global__ __launch_bounds__(kNT, D > 128 ? 1 : 2) void flash_bf16_kernel(SdpaPa
       if (odd || ragged) place_runs(mk, mrow, kb + half * 8, Tk, odd, ragged);
       off = runs_all_off(mk);
     }
+    // kAnyMask: the tile's values, all in flight at once under the products,
+    // in steps of 16 keys up to the row's end.  Loaded where each was used,
+    // behind a branch on the type and waited for alone, past the row's end
+    // too, they took 9.8 us a call on [1,8,300,64] with 7 keys (bf16 mask) and
+    // 65 on [1,16,1024,64] GQA with strided keys (f32); 6.0 and 38 here.
+    float any[MT == kAnyMask ? kMT * 16 : 1] = {};
+    if constexpr (MT == kAnyMask) {
+      auto rd = [&](auto mt_tag) __attribute__((always_inline)) {
+#pragma unroll
+        for (int g = 0; g < kKS; ++g)
+          if (!EDGE || g == 0 || kb + g * 16 < Tk)
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+              any[g * 8 + i] = load_mask_t<decltype(mt_tag)::value>(
+                  p.mask, moff + min(kb + g * 16 + half * 8 + i, Tk - 1) * p.ms[3]);
+      };
+      if (p.mask_dtype == MFX_F32) rd(std::integral_constant<int, 1>{});
+      else if (p.mask_dtype == MFX_BF16) rd(std::integral_constant<int, 2>{});
+      else rd(std::integral_constant<int, 3>{});
+    }
     f32x16 s[kMT];
     float mx = -INFINITY;
     if (!off) {
@@ -238,7 +258,7 @@ __global__ __launch_bounds__(kNT, D > 128 ? 1 : 2) void flash_bf16_kernel(SdpaPa
         float x = s[mt][i];
         const int g = mt * 2 + (i >> 3), key = kb + g * 16 + half * 8 + (i & 7);
         if constexpr (MT == kAnyMask) {
-          x = x * sl2 + mask_log2(load_mask(p.mask, p.mask_dtype, moff + min(key, Tk - 1) * p.ms[3]));
+          x = x * sl2 + mask_log2(any[g * 8 + (i & 7)]);
         } else if constexpr (MASK) {
           Run& run = mk[AHEAD ? g : 0];
           if constexpr (!AHEAD)

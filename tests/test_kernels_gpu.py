@@ -775,7 +775,7 @@ def test_sdpa_finite_mask_fully_masked_rows(cuda, nat, oracle, case, mdt):
 @pytest.mark.parametrize("D", [32, 64, 96, 128, 256])
 @pytest.mark.parametrize("tq,tk,form", [
     (33, 8, "dense"), (65, 71, "dense"), (40, 64, "dense"), (130, 199, "dense"), (70, 130, "off_by_one"),
-    (40, 7, "dense"), (40, 90, "columns"), (40, 90, "row_constant"), (300, 333, "band")])
+    (40, 7, "dense"), (40, 17, "columns"), (40, 90, "columns"), (40, 90, "row_constant"), (300, 333, "band")])
 def test_sdpa_query_varying_mask_runs(cuda, nat, oracle, dt, mdt, D, tq, tk, form):
     """Masks that vary along query rows: read in runs of eight keys (rows that
     start on and off a dword, ends short of a run and of a tile, a base one
