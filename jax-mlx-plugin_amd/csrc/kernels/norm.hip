@@ -4,8 +4,8 @@
 // A row is owned by 16 or 64 lanes of one wavefront (rows up to 1024
 // 16-byte vectors, i.e. 4096 f32 / 8192 bf16 or f16 elements) or by a 256-thread
 // workgroup (up to 4096 vectors); unaligned rows and rows of up to 64 Ki
-// elements take row_kernel_any (up to 1024 threads a row), longer ones a
-// looped fallback.  Each element is read from HBM once and written once -- the HBM
+// elements take row_kernel_any (up to 1024 threads a row), longer ones and
+// small calls on short unaligned rows a looped kernel.  Each element is read from HBM once and written once -- the HBM
 // roofline's algorithmic traffic.
 #include "rowvec.h"
 
@@ -235,9 +235,9 @@ __global__ __launch_bounds__(LANES > kBlock ? LANES : kBlock) void row_kernel_an
   }
 }
 
-// Fallback for rows longer than the register-resident variants (and
-// parameters of a type those do not take): one workgroup per row, scalar
-// strided loops, three passes over the row.
+// Rows longer than the register-resident variants, parameters of a type those
+// do not take, and small calls on short unaligned rows (looped_first): one
+// workgroup per row, scalar strided loops, three passes over the row.
 template <typename T, RowOp OP>
 __global__ __launch_bounds__(kBlock) void row_kernel_looped(
     const T* __restrict__ x, T* __restrict__ y, const void* __restrict__ gamma,
@@ -346,6 +346,24 @@ int dispatch_any(const mfx_norm_args& a, hipStream_t s) {
   return fail(MFX_E_INVALID, "row too long for row_kernel_any");  // (excluded by kAnyMax)
 }
 
+// Whether a call on short unaligned rows is too small for row_kernel_any: while
+// the looped kernel's workgroups, one a row, are on the chip together, a call is
+// one row's latency, and there an element a load in 256 threads beats runs of
+// eight in a wavefront, whose last run reads its elements behind their
+// conditions.  16-bit rows, looped against runs in us: LayerNorm of 64 rows of
+// 31 3.5 and 4.9, of 512 rows of 767 5.0 and 5.9, of 2048 rows of 101 both 4.6;
+// softmax, which holds its row for one pass less, 256 rows of 767 4.1 and 4.4,
+// 1024 rows of 511 4.2 and 4.0, 4096 rows of 310 6.9 and 4.5.  RMSNorm, whose
+// looped kernel reads a row once less, has it at longer rows (64 of 2047: 5.6
+// and 6.2), and in f32 (64 rows of 63: 3.1 and 3.4) below 512 rows.
+template <typename T, RowOp OP>
+bool looped_first(const mfx_norm_args& a) {
+  constexpr bool RMS = OP == RowOp::kRmsNorm;
+  if (a.n > (RMS && sizeof(T) == 2 ? 2048 : 1024) || (sizeof(T) == 4 && !RMS)) return false;
+  const int64_t cus = device_cu_count();
+  return sizeof(T) == 4 ? a.rows <= 2 * cus : a.rows <= 8 * cus && a.rows * a.n <= (is_softmax(OP) ? 768 : RMS ? 3072 : 2048) * cus;
+}
+
 template <typename T, RowOp OP>
 int dispatch_typed(const mfx_norm_args& a, hipStream_t s) {
   constexpr int VEC = Vec16<T>::N;
@@ -369,7 +387,7 @@ int dispatch_typed(const mfx_norm_args& a, hipStream_t s) {
     }
     return dispatch_vec<T, float, OP>(a, s, nvec);
   }
-  if (a.n <= kAnyMax<OP> && pvec) {
+  if (a.n <= kAnyMax<OP> && pvec && !looped_first<T, OP>(a)) {
     if (params && a.param_dtype != MFX_F32) {
       if constexpr (kF16) return dispatch_any<T, _Float16, OP>(a, s);
       else return dispatch_any<T, bf16, OP>(a, s);

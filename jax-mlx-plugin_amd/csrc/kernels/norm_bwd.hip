@@ -358,11 +358,11 @@ __global__ __launch_bounds__(LANES > kBlock ? LANES : kBlock) void ln_bwd_rows_a
   }
 }
 
-// Rows longer than the register-resident variants (and parameters of a type
-// those do not take): the
-// workgroup walks rows blockIdx.x, blockIdx.x + G, ...; thread t owns columns
-// t, t + 256, ... of the block's partial rows, which it updates in place
-// (no other thread touches them).
+// Rows longer than the register-resident variants, parameters of a type those
+// do not take, and small unaligned calls (plan_bwd): the workgroup walks rows
+// blockIdx.x, blockIdx.x + G, ...; thread t owns columns t, t + 256, ... of the
+// block's partial rows, which it updates in place (no other thread touches
+// them).
 template <typename T>
 __global__ __launch_bounds__(kBlock) void ln_bwd_rows_looped(
     const T* __restrict__ x, const T* __restrict__ dy, T* __restrict__ dx,
@@ -471,7 +471,13 @@ BwdPlan plan_bwd(const mfx_norm_bwd_args& a) {
   // Aligned rows of up to 256 lanes run ln_bwd_rows; ln_bwd_rows_any starts
   // at a wavefront per row.
   static const int kLanes[5] = {16, 64, 256, 512, 1024};
-  for (int li = 0; li < 5 && !p.vector && ptype; ++li) {
+  // Unaligned calls that are one row's latency take the looped kernel: a single
+  // row of up to 1024 elements (one row in ln_bwd_rows_any's pair; 63 bf16
+  // elements 6.0 against 8.2 us, 767 of f32 7.9 and 9.1), and few rows of up to
+  // 256 16-bit elements, whose last run waits for its elements one by one (64
+  // rows of 31: 8.6 and 9.7; of 310: 10.5 and 9.8; 256 rows of 63: 10.2 and 10.0).
+  const bool looped = !aligned && (a.rows == 1 ? a.n <= 1024 : a.dtype != MFX_F32 && a.rows <= 128 && a.n <= 256);
+  for (int li = 0; li < 5 && !p.vector && ptype && !looped; ++li) {
     p.any = !aligned || li >= 3;
     if (p.any && li == 0) continue;
     for (int nv = li >= 3 ? maxnv : 1; nv <= maxnv; nv *= 2)

@@ -85,16 +85,18 @@ def test_layer_norm_strided_rows_and_constant_rows(cuda, nat, oracle):
 
 
 @pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
-@pytest.mark.parametrize("n", [1, 3, 255, 257, 511, 1025, 2049, 4099, 8193, 16385, 32767, 32769, 65535, 65537])
-def test_rows_of_any_length_and_alignment(cuda, nat, oracle, dt, n):
+@pytest.mark.parametrize("rows,n", [(5, n) for n in (1, 3, 255, 257, 511, 1025, 2049, 4099, 8193, 16385, 32767, 32769,
+                                                     65535, 65537)]
+                         + [(2100, n) for n in (1, 3, 255, 257, 511, 513, 1023, 1025)] + [(300, 2047)])
+def test_rows_of_any_length_and_alignment(cuda, nat, oracle, dt, rows, n):
     """LayerNorm, RMSNorm, softmax and log-softmax on rows off 16 bytes, at the
-    edges of the lanes-per-row variants and past the register-resident ones:
+    edges of the lanes-per-row variants and past the register-resident ones, in
+    calls small enough for the looped kernel at short rows and past that line:
     contiguous odd rows, and a view one element in with padded rows.  f32 bar:
     the norms'; sums of n terms add at most n * 2^-24 relative to their size,
     split over at least 64 lanes."""
     td = {"f32": cuda.float32, "bf16": cuda.bfloat16, "f16": cuda.float16}[dt]
     rng = np.random.default_rng(n)
-    rows = 5
     x = rng.standard_normal((rows, n)) * 2 + 0.5
     flat = cuda.zeros(1 + rows * (n + 3), dtype=td, device="cuda")
     view = flat[1:].view(rows, n + 3)[:, :n]
@@ -185,7 +187,8 @@ def test_layer_norm_bwd_without_gamma_strided_and_empty(cuda, nat, oracle):
 @pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
 @pytest.mark.parametrize("rows,n", [
     (9, 1), (9, 3), (8, 255), (9, 257), (9, 511), (9, 513), (9, 1025), (9, 2049), (9, 4097), (9, 4104), (9, 8191),
-    (9, 8200), (9, 16383), (9, 16384), (9, 16385), (8300, 33), (2100, 1031)])
+    (9, 8200), (9, 16383), (9, 16384), (9, 16385), (8300, 33), (2100, 1031),
+    (1, 1), (1, 1023), (1, 1025), (2, 1023), (128, 255), (129, 255), (200, 1), (200, 7)])
 def test_layer_norm_bwd_rows_of_any_length_and_alignment(cuda, nat, oracle, dt, rows, n):
     """Rows off 16 bytes, at the edges of the threads-per-row variants and past
     the longest, as a contiguous tensor and as views one element in; groups
