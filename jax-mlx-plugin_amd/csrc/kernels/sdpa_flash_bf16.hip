@@ -118,11 +118,12 @@ __global__ __launch_bounds__(kNT, D > 128 ? 1 : 2) void flash_bf16_kernel(SdpaPa
   constexpr bool AHEAD = RUNS && D <= 128;
   constexpr bool FENCE = D > 128;
   // Head sizes 32 and 96: the per-row kernel, which these calls took before,
-  // keeps probabilities in fp32, so here they enter PV as two 16-bit terms,
-  // to 2^-17 of a row's largest or better: with a bf16 bias at 2048 keys the
-  // output is 1.66e-3 (2-norm) from its 64-bit value, all of it the output's
-  // own rounding, as the per-row kernel's is (one term: 2.3e-3).  [4,16,2048,D]
-  // takes 132 (D = 32) and 204 us (D = 96), against 10.2 and 17.0 ms there.
+  // keeps probabilities in fp32, so here they enter PV as three 16-bit terms,
+  // which hold all 24 bits of each (f16: to 2^-25 of the row's largest): the
+  // output's error is its own rounding, as the per-row kernel's is (1.66e-3 in
+  // 2-norm with a bf16 bias at 2048 keys; with one term 2.3e-3), and where V
+  // cancels in the sum it is fp32's.  [4,16,2048,D] takes 157 (D = 32) and 237 us
+  // (D = 96), against 10.2 and 17.0 ms there (with two terms 140 and 218).
   constexpr bool SPLIT = DV != D;
   using Run = MaskRun<RUNS ? MT : 1>;
   Run mk[AHEAD ? kKS : 1];
@@ -323,30 +324,18 @@ __global__ __launch_bounds__(kNT, D > 128 ? 1 : 2) void flash_bf16_kernel(SdpaPa
       return MASK ? __builtin_amdgcn_exp2f(s[mt][i] + nbase) : __builtin_amdgcn_exp2f(fmaf(s[mt][i], sl2, nbase));
     };
     // P rounded to the element type and the row sum of exactly the rounded
-    // values the PV product consumes, two per instruction.
-    bf16x8 pb[kKS], pl[SPLIT ? kKS : 1];
+    // values the PV product consumes, two per instruction.  (SPLIT: P stays in
+    // s until its step of the product.)
+    bf16x8 pb[SPLIT ? 1 : kKS];
     float l0 = 0.f, l1 = 0.f;
     if constexpr (SPLIT) {
-      // hi + lo, and the row sum of the values before the rounding.
-      u32x4 hw[kKS], lw[kKS];
 #pragma unroll
       for (int mt = 0; mt < kMT; ++mt)
 #pragma unroll
-        for (int i = 0; i < 16; i += 2) {
-          const float p0 = pexp(mt, i), p1 = pexp(mt, i + 1);
-          const uint32_t w = pack2<E>(p0, p1);
-          const float h0 = E == 0 ? __uint_as_float(w << 16) : f16_lo(w);
-          const float h1 = E == 0 ? __uint_as_float(w & 0xFFFF0000u) : f16_hi(w);
-          hw[mt * 2 + (i >> 3)][(i & 7) >> 1] = w;
-          lw[mt * 2 + (i >> 3)][(i & 7) >> 1] = pack2<E>(p0 - h0, p1 - h1);
-          l0 += p0;
-          l1 += p1;
+        for (int i = 0; i < 16; ++i) {
+          s[mt][i] = pexp(mt, i);
+          (i & 1 ? l1 : l0) += s[mt][i];
         }
-#pragma unroll
-      for (int j = 0; j < kKS; ++j) {
-        pb[j] = __builtin_bit_cast(bf16x8, hw[j]);
-        pl[SPLIT ? j : 0] = __builtin_bit_cast(bf16x8, lw[j]);
-      }
     } else if constexpr (E == 0) {
 #pragma unroll
       for (int mt = 0; mt < kMT; ++mt)
@@ -380,20 +369,48 @@ __global__ __launch_bounds__(kNT, D > 128 ? 1 : 2) void flash_bf16_kernel(SdpaPa
     l_run += l0 + l1;
     if constexpr (FENCE) fence();
     __builtin_amdgcn_s_setprio(3);
-#pragma unroll
-    for (int dt = 0; dt < DV / 32; ++dt)
+    // k-slots 0-3: keys ks*16 + 8*half + e; slots 4-7: the same + 4.
+    auto v_frag = [&](int ks, int dt) __attribute__((always_inline)) {
+      const char* v_rows = vb8 + ks * 16 * D * 2;
+      const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(v_rows + (va ^ dt * 64)));
+      const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(v_rows + (va4 ^ dt * 64)));
+      return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+    if constexpr (SPLIT) {
 #pragma unroll
       for (int ks = 0; ks < kKS; ++ks) {
-        // k-slots 0-3: keys ks*16 + 8*half + e; slots 4-7: the same + 4.
-        const char* v_rows = vb8 + ks * 16 * D * 2;
-        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(v_rows + (va ^ dt * 64)));
-        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(v_rows + (va4 ^ dt * 64)));
-        const bf16x8 a = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-        o[dt] = mfma16<E>(a, pb[ks], o[dt]);
-        if constexpr (SPLIT) o[dt] = mfma16<E>(a, pl[SPLIT ? ks : 0], o[dt]);
-        if constexpr (FENCE)
-          if ((ks & 1) == 1) fence();
+        bf16x8 term[3];
+        float rest[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) rest[j] = s[ks >> 1][(ks & 1) * 8 + j];
+#pragma unroll
+        for (int n = 0; n < 3; ++n) {
+          u32x4 w;
+#pragma unroll
+          for (int j = 0; j < 8; j += 2) {
+            w[j >> 1] = pack2<E>(rest[j], rest[j + 1]);
+            rest[j] -= E == 0 ? __uint_as_float(w[j >> 1] << 16) : f16_lo(w[j >> 1]);
+            rest[j + 1] -= E == 0 ? __uint_as_float(w[j >> 1] & 0xFFFF0000u) : f16_hi(w[j >> 1]);
+          }
+          term[n] = __builtin_bit_cast(bf16x8, w);
+        }
+#pragma unroll
+        for (int dt = 0; dt < DV / 32; ++dt) {
+          const bf16x8 a = v_frag(ks, dt);
+#pragma unroll
+          for (int n = 0; n < 3; ++n) o[dt] = mfma16<E>(a, term[n], o[dt]);
+        }
       }
+    } else {
+#pragma unroll
+      for (int dt = 0; dt < DV / 32; ++dt)
+#pragma unroll
+        for (int ks = 0; ks < kKS; ++ks) {
+          o[dt] = mfma16<E>(v_frag(ks, dt), pb[ks], o[dt]);
+          if constexpr (FENCE)
+            if ((ks & 1) == 1) fence();
+        }
+    }
     if constexpr (FENCE) fence();
   };
 

@@ -819,10 +819,9 @@ def test_sdpa_query_varying_mask_runs(cuda, nat, oracle, dt, mdt, D, tq, tk, for
 @pytest.mark.parametrize("D", [32, 96])
 @pytest.mark.parametrize("tq,tk", [(70, 7), (130, 199), (256, 1024)])
 def test_sdpa_query_varying_mask_keeps_fp32_probabilities(cuda, nat, oracle, dt, D, tq, tk):
-    """At head sizes 32 and 96 P enters PV as two 16-bit terms: beside the
-    output's own rounding (2-norm 2^-9.2 of it in bf16, 2^-12.2 in f16) its
-    error of 2^-17 (f16: 2^-22) is lost, where one term would add as much
-    again."""
+    """At head sizes 32 and 96 P enters PV as three 16-bit terms, all its bits:
+    beside the output's own rounding (2-norm 2^-9.2 of it in bf16, 2^-12.2 in
+    f16) its error is lost, where one term would add as much again."""
     td = {"bf16": cuda.bfloat16, "f16": cuda.float16}[dt]
     q, k, v = make_qkv(cuda, 64, (2, 2, tq, D), (2, 1, tk, D), td)
     m = dev(cuda, np.random.default_rng(65).standard_normal((1, 2, tq, tk)), td)
@@ -830,6 +829,36 @@ def test_sdpa_query_varying_mask_keeps_fp32_probabilities(cuda, nat, oracle, dt,
     ref = oracle.sdpa(host(q), host(k), host(v), D ** -0.5, mask=np.broadcast_to(host(m), (2, 2, tq, tk)).copy())
     rounded = host(cuda.from_numpy(ref).to(td))
     assert np.linalg.norm(out - ref) <= 1.05 * np.linalg.norm(rounded - ref)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("D", [32, 96])
+@pytest.mark.parametrize("tk", [7, 64, 130])
+def test_sdpa_query_varying_mask_probabilities_keep_all_bits(cuda, nat, dt, D, tk):
+    """Head sizes 32 and 96, where V cancels in the sum: one key of probability
+    p (before the division) against three of 1 whose values add up to -p to 24
+    bits, so the output is p's error alone.  Bar: 2^-22 of p before the
+    division, four roundings to fp32 (p's exponent, the exponential, the sum);
+    p in two bf16 terms is off by up to 2^-18."""
+    td = {"bf16": cuda.bfloat16, "f16": cuda.float16}[dt]
+    H, tq, scale = 64, 40, 256.0
+    b = np.random.default_rng(D).uniform(-0.69, -0.01, H).astype(np.float32)
+    p = np.exp(b.astype(np.float64))
+    v = np.zeros((1, H, tk, D))
+    rest = p.copy()
+    for j in range(3):
+        x = host(cuda.from_numpy(rest).to(td))
+        v[0, :, j] = -x[:, None] * scale
+        rest -= x
+    v[0, :, 3] = scale
+    m = np.full((1, H, tq, tk), -np.inf, np.float32)
+    m[..., :3] = 0
+    m[..., 3] = b[None, :, None]
+    q = cuda.zeros(1, H, tq, D, dtype=td, device="cuda")
+    k = cuda.zeros(1, H, tk, D, dtype=td, device="cuda")
+    out = host(nat.sdpa(q, k, dev(cuda, v, td), mask=dev(cuda, m, cuda.float32)))
+    err = np.abs(out - (rest * scale / (3 + p))[None, :, None, None]) * ((3 + p) / scale)[None, :, None, None]
+    assert err.max() <= 2.0 ** -22
 
 
 @pytest.mark.parametrize("D", [64, 128, 256])
