@@ -131,6 +131,39 @@ def test_lds_wait_check_names_the_early_read(case):
         native_build._check_lds_waits(Path("k.hip"), _kernel(body))
 
 
+@pytest.mark.parametrize("note,lost", [
+    ("; kill: def $vgpr4 killed $vgpr9 killed $exec", True),
+    ("; kill: def $agpr4 killed $vgpr4 killed $exec", True),
+    ("; kill: def $vgpr4 killed $vgpr4 killed $exec", False),
+    ("; kill: def $vgpr4_vgpr5 killed $vgpr4_vgpr5 def $vgpr4_vgpr5_vgpr6", False)])
+def test_lost_copy_check(note, lost):
+    asm = _kernel(f"""
+        v_mov_b32_e32 v1, 0
+        {note}
+        v_add_f32_e32 v1, v4, v1""")
+    if lost:
+        with pytest.raises(RuntimeError, match="k.hip:\na lost register copy: kill: def"):
+            native_build._check_lost_copies(Path("k.hip"), asm)
+    else:
+        native_build._check_lost_copies(Path("k.hip"), asm)
+
+
+@pytest.mark.parametrize("name", ["sdpa_bwd_f32.hip", "gemm16.hip"])
+def test_lost_copy_check_runs_on_every_kernel_file(monkeypatch, tmp_path, name):
+    """The assembly of a file with and without inline-asm LDS reads: a compiler
+    stand-in writes one lost copy, and the build refuses the file."""
+    cc = tmp_path / "hipcc"
+    cc.write_text("""#!/bin/sh
+for a; do last=$a; done
+echo '\t; kill: def $vgpr4 killed $vgpr9' > "$last" 2>/dev/null
+""")
+    cc.chmod(0o755)
+    monkeypatch.setattr(native_build, "HIPCC", str(cc))
+    monkeypatch.setattr(native_build, "_RESOURCE_REMARK", str(tmp_path / "remark"))
+    with pytest.raises(RuntimeError, match=f"{name}:\na lost register copy"):
+        native_build._compile_hip(native_build.CSRC / "kernels" / name, tmp_path / (Path(name).stem + ".o"))
+
+
 def test_lds_wait_check_runs_on_the_built_kernels():
     """The build writes each guarded file's device assembly beside its object
     and checks it; the built assembly holds the kernels and passes."""
