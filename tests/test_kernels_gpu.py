@@ -13,6 +13,7 @@ pytestmark = pytest.mark.gpu
 
 F32_NORM_TOL = 1e-5
 F32_SDPA_TOL = 1e-4
+F32_BWD_TOL = 1e-5  # the fp32 matrix-core backward, of the largest value (at least 1)
 BF16_REL_TOL = 2e-2
 F16_REL_TOL = 5e-3  # as in test_f16_gpu.py
 
@@ -92,10 +93,15 @@ def test_rows_of_any_length_and_alignment(cuda, nat, oracle, dt, rows, n):
     """LayerNorm, RMSNorm, softmax and log-softmax on rows off 16 bytes, at the
     edges of the lanes-per-row variants and past the register-resident ones, in
     calls small enough for the looped kernel at short rows and past that line:
-    contiguous odd rows, and a view one element in with padded rows.  f32 bar:
-    the norms'; sums of n terms add at most n * 2^-24 relative to their size,
-    split over at least 64 lanes."""
+    contiguous odd rows, and a view one element in with padded rows; outputs
+    one element into a filled buffer.  Bars, per element: half an ulp of the
+    output's type (24, 8 and 11 bits: 2^-24, 2^-8, 2^-11 of its value; f16
+    subnormals 2^-25), and
+    the fp32 work behind it, for the norms and log-softmax F32_NORM_TOL of the
+    largest value, for softmax 2e-5 of the element (exponents of up to 20 to
+    2^-24 each twice, sums of at most 256 terms a lane to 2^-24 a term)."""
     td = {"f32": cuda.float32, "bf16": cuda.bfloat16, "f16": cuda.float16}[dt]
+    rounding = {"f32": 2.0 ** -24, "bf16": 2.0 ** -8, "f16": 2.0 ** -11}[dt]
     rng = np.random.default_rng(n)
     x = rng.standard_normal((rows, n)) * 2 + 0.5
     flat = cuda.zeros(1 + rows * (n + 3), dtype=td, device="cuda")
@@ -104,18 +110,23 @@ def test_rows_of_any_length_and_alignment(cuda, nat, oracle, dt, rows, n):
     g, b = dev(cuda, 1 + 0.1 * rng.standard_normal(n), td), dev(cuda, 0.1 * rng.standard_normal(n), td)
     for xd in (dev(cuda, x, td), view):
         xh = host(xd)
-        out = cuda.full((1 + rows * (n + 2),), 7.0, dtype=td, device="cuda")
-        ov = out[1:].view(rows, n + 2)[:, :n]
-        for got, ref in ((nat.layer_norm(xd, g, b, out=ov), oracle.layer_norm(xh, host(g), host(b), 1e-5)),
-                         (nat.rms_norm(xd, g), oracle.rms_norm(xh, host(g), 1e-5)),
-                         (nat.softmax(xd), oracle.softmax(xh)), (nat.log_softmax(xd), oracle.log_softmax(xh))):
-            got = host(got)
-            if dt == "f32":
-                assert np.abs(got - ref).max() <= F32_NORM_TOL * max(1.0, np.abs(ref).max())
+        for name, op, ref in (
+                ("layer_norm", lambda o: nat.layer_norm(xd, g, b, out=o), oracle.layer_norm(xh, host(g), host(b), 1e-5)),
+                ("rms_norm", lambda o: nat.rms_norm(xd, g, out=o), oracle.rms_norm(xh, host(g), 1e-5)),
+                ("softmax", lambda o: nat.softmax(xd, out=o), oracle.softmax(xh)),
+                ("log_softmax", lambda o: nat.log_softmax(xd, out=o), oracle.log_softmax(xh))):
+            out = cuda.full((1 + rows * (n + 2),), 7.0, dtype=td, device="cuda")
+            ov = out[1:].view(rows, n + 2)[:, :n]
+            got = host(op(ov))
+            if name == "softmax":
+                bar = rounding * ref + 2e-5 * ref + (2.0 ** -25 if dt == "f16" else 0)
+                sums = np.abs(got.sum(-1) - 1).max()
+                assert sums <= rounding + 2e-5 + (n * 2.0 ** -25 if dt == "f16" else 0), sums
             else:
-                assert np.abs(got - ref).max() <= BF16_REL_TOL * max(np.abs(ref).max(), 1e-3)
-        pad = out[1:].view(rows, n + 2)[:, n:]
-        assert bool((pad == 7).all()) and float(out[0]) == 7.0  # nothing written beside the rows
+                bar = rounding * np.abs(ref) + F32_NORM_TOL * max(1.0, np.abs(ref).max())
+            assert (np.abs(got - ref) <= bar).all(), (name, (np.abs(got - ref) - bar).max())
+            pad = out[1:].view(rows, n + 2)[:, n:]
+            assert bool((pad == 7).all()) and float(out[0]) == 7.0  # nothing written beside the rows
 
 
 # ------------------------------------------------------- LayerNorm backward
@@ -213,7 +224,7 @@ def test_layer_norm_bwd_rows_of_any_length_and_alignment(cuda, nat, oracle, dt, 
                 assert np.abs(o - r).max() <= max(F32_NORM_TOL, terms * 2.0 ** -24) * max(1.0, np.abs(r).max())
         else:
             for o, r in zip(outs, ref):
-                assert np.abs(o - r).max() <= BF16_REL_TOL * max(np.abs(r).max(), 1e-3)
+                assert np.abs(o - r).max() <= (BF16_REL_TOL if dt == "bf16" else F16_REL_TOL) * max(np.abs(r).max(), 1e-3)
 
 
 @pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
@@ -304,7 +315,7 @@ def check_sdpa(out, ref, dtype):
         assert err <= F32_SDPA_TOL, err
     else:
         r = rel_inf(out, ref)
-        assert r <= BF16_REL_TOL, r
+        assert r <= (F16_REL_TOL if dtype == "f16" else BF16_REL_TOL), r
 
 
 @pytest.mark.parametrize("causal", [False, True])
@@ -812,7 +823,7 @@ def test_sdpa_query_varying_mask_runs(cuda, nat, oracle, dt, mdt, D, tq, tk, for
     assert nat.sdpa_kernel_name(q, k, v, mask=maskd) == f"flash_{dt}_d{D}"
     a = nat.sdpa(q, k, v, scale=D ** -0.5, mask=maskd, causal=causal)
     ref = oracle.sdpa(host(q), host(k), host(v), D ** -0.5, causal=causal, mask=host(maskd))
-    check_sdpa(a, ref, "bf16")
+    check_sdpa(a, ref, dt)
 
 
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
@@ -904,15 +915,15 @@ def test_sdpa_decode_mfma_fully_masked_row_is_nan(cuda, nat):
 # ||d - ref||_inf <= 1e-4 * max(1, ||ref||_inf) per gradient; bf16: the
 # relative bar on each of dq, dk, dv.
 
-def check_grads(outs, refs, dtype):
+def check_grads(outs, refs, dtype, f32_tol=F32_SDPA_TOL):
     for name, o, r in zip(("dq", "dk", "dv"), outs, refs):
         o = host(o)
         if dtype == "f32":
             err = np.abs(o - r).max()
-            assert err <= F32_SDPA_TOL * max(1.0, np.abs(r).max()), (name, err)
+            assert err <= f32_tol * max(1.0, np.abs(r).max()), (name, err)
         else:
             rr = rel_inf(o, r)
-            assert rr <= BF16_REL_TOL, (name, rr)
+            assert rr <= (F16_REL_TOL if dtype == "f16" else BF16_REL_TOL), (name, rr)
 
 
 def bwd_case(cuda, nat, oracle, seed, qshape, kshape, dtype, *, causal=False, scale=None, mask=None,
@@ -1024,7 +1035,7 @@ def test_sdpa_bwd_query_varying_mask_runs(cuda, nat, oracle, dt, mdt, D, tq, tk,
     causal = form == "causal"
     grads = nat.sdpa_bwd(q, k, v, g, causal=causal, mask=maskd)
     refs = oracle.sdpa_bwd(host(q), host(k), host(v), host(g), D ** -0.5, causal=causal, mask=host(maskd))
-    check_grads(grads, refs, "bf16")
+    check_grads(grads, refs, dt)
 
 
 @pytest.mark.parametrize("rows", [1, 64])
@@ -1058,8 +1069,9 @@ def test_sdpa_bwd_odd_head_size_generic(cuda, nat, oracle):
 ])
 def test_sdpa_bwd_f32_matrix_cores(cuda, nat, oracle, D, B, hq, hkv, tq, tk, causal, mdt, layout):
     """The fp32 matrix-core backward at tile edges, every mask type, GQA and
-    both workgroup sizes.  Bar as the other f32 cases'; the accumulation
-    bound (D + T) * 2^-23 * sum|terms| stays below it at these sizes."""
+    both workgroup sizes.  Bar F32_BWD_TOL: these sums of D + T terms rounded
+    to 2^-24 each are up to 1.0e-6 from their 64-bit values, and another order
+    of them moves by as much."""
     shape = (lambda h, t: (B, h, t, D)) if layout == "bhtd" else (lambda h, t: (B, t, h, D))
     mask = None
     if mdt:
@@ -1075,12 +1087,12 @@ def test_sdpa_bwd_f32_matrix_cores(cuda, nat, oracle, D, B, hq, hkv, tq, tk, cau
         whole = nat.sdpa_bwd(q, k, v, go, causal=causal)
         part = nat.sdpa_bwd(*(t[5:6].contiguous() for t in (q, k, v, go)), causal=causal)
         refs = oracle.sdpa_bwd(*(host(t[5:6]) for t in (q, k, v, go)), 1.0 / np.sqrt(D), causal=causal, mask=None)
-        check_grads([t[5:6] for t in whole], refs, "f32")
-        check_grads(part, refs, "f32")
+        check_grads([t[5:6] for t in whole], refs, "f32", F32_BWD_TOL)
+        check_grads(part, refs, "f32", F32_BWD_TOL)
         return
     grads, refs = bwd_case(cuda, nat, oracle, 300 + D, shape(hq, tq), shape(hkv, tk), "f32", causal=causal, mask=mask,
                            layout=layout)
-    check_grads(grads, refs, "f32")
+    check_grads(grads, refs, "f32", F32_BWD_TOL)
 
 
 @pytest.mark.parametrize("D", [32, 64, 96, 128])
@@ -1095,7 +1107,7 @@ def test_sdpa_bwd_f32_hidden_rows_that_are_not_finite(cuda, nat, D, B, hq, hkv, 
     """A NaN or an infinity in a row that causality hides from a query (or
     key) does not reach its gradient, also from the same tile, and reaches
     those that see it as on the per-row kernels (the same call with rows off
-    16 bytes).  Finite values: the other f32 cases' bar."""
+    16 bytes).  Finite values: F32_BWD_TOL."""
     g = cuda.Generator(device="cuda").manual_seed(D + tk)
     q, k, v, go = (cuda.randn(B, h, t, D, generator=g, device="cuda")
                    for h, t in ((hq, tq), (hkv, tk), (hkv, tk), (hq, tq)))
@@ -1118,7 +1130,7 @@ def test_sdpa_bwd_f32_hidden_rows_that_are_not_finite(cuda, nat, D, B, hq, hkv, 
         assert np.array_equal(np.isfinite(a), np.isfinite(b)), name
         odd = ~np.isfinite(b)
         assert np.array_equal(a[odd], b[odd], equal_nan=True), name
-        assert np.abs(a[~odd] - b[~odd]).max(initial=0) <= F32_SDPA_TOL * np.abs(b[~odd]).max(initial=1), name
+        assert np.abs(a[~odd] - b[~odd]).max(initial=0) <= F32_BWD_TOL * np.abs(b[~odd]).max(initial=1), name
     if rows and which == "k":
         assert bool(cuda.isfinite(got[0][:, :, :min(rows)]).all())
     if rows and which == "g":
@@ -1138,7 +1150,7 @@ def test_sdpa_bwd_f32_unaligned_rows(cuda, nat, oracle):
     refs = nat.sdpa_bwd(q, k, v, g)
     assert nat.sdpa_bwd_kernel_name(q, wide[..., :D], v) == "generic"
     for a, r in zip(nat.sdpa_bwd(q, wide[..., :D], v, g), refs):
-        assert np.abs(host(a) - host(r)).max() <= F32_SDPA_TOL * max(1.0, np.abs(host(r)).max())
+        assert np.abs(host(a) - host(r)).max() <= F32_BWD_TOL * max(1.0, np.abs(host(r)).max())
     v1 = v[:, :, :1].expand(B, H, T, D)
     assert nat.sdpa_bwd_kernel_name(q, k, v1) == "generic"
     dense = nat.sdpa_bwd(q, k, v1.contiguous(), g)
@@ -1146,7 +1158,7 @@ def test_sdpa_bwd_f32_unaligned_rows(cuda, nat, oracle):
     a = nat.sdpa_bwd_args(q, k, v1, g, dq, dk, dv)
     nat.check(nat.load().mfx_sdpa_bwd(ctypes.byref(a), ctypes.c_void_p(cuda.cuda.current_stream().cuda_stream)))
     for o, r in zip((dq, dk, dv), dense):
-        assert np.abs(host(o) - host(r)).max() <= F32_SDPA_TOL * max(1.0, np.abs(host(r)).max())
+        assert np.abs(host(o) - host(r)).max() <= F32_BWD_TOL * max(1.0, np.abs(host(r)).max())
 
 
 @pytest.mark.parametrize("over", ["q", "g"])
@@ -1154,7 +1166,7 @@ def test_sdpa_bwd_f32_unaligned_rows(cuda, nat, oracle):
 @pytest.mark.parametrize("D,causal", [(32, False), (64, True), (96, True), (128, False)])
 def test_sdpa_bwd_f32_dq_in_place(cuda, nat, D, causal, saved, over):
     """dq stored over q or dO row by row: the gradients of the call with
-    outputs of its own (the other f32 cases' bar)."""
+    outputs of its own (within F32_BWD_TOL)."""
     import ctypes
 
     gen = cuda.Generator(device="cuda").manual_seed(D)
@@ -1169,7 +1181,7 @@ def test_sdpa_bwd_f32_dq_in_place(cuda, nat, D, causal, saved, over):
     a = nat.sdpa_bwd_args(q, k, v, g, dq, dk, dv, **kw)
     nat.check(nat.load().mfx_sdpa_bwd(ctypes.byref(a), cuda.cuda.current_stream().cuda_stream))
     for name, o, r in zip(("dq", "dk", "dv"), (dq, dk, dv), refs):
-        assert np.abs(host(o) - host(r)).max() <= F32_SDPA_TOL * max(1.0, np.abs(host(r)).max()), name
+        assert np.abs(host(o) - host(r)).max() <= F32_BWD_TOL * max(1.0, np.abs(host(r)).max()), name
 
 
 def test_sdpa_bwd_known_answers(cuda, nat):
