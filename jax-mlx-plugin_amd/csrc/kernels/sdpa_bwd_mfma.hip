@@ -69,8 +69,6 @@ enum BwdPhaseSlot {
   kPhX, kPhYV, kPhSync, kPhVmwait, kPhBarrier, kPhLast, kPhBlocks, kPhEdges, kPhTiles,
   kPhRtStart, kPhCStart, kPhRtLoop, kPhCLoop, kPhCEpi, kBwdPhaseSlots
 };
-__device__ __forceinline__ unsigned ph_now() { return (unsigned)__builtin_amdgcn_s_memtime(); }
-__device__ __forceinline__ unsigned ph_real() { return (unsigned)__builtin_amdgcn_s_memrealtime(); }
 #endif
 
 namespace {
@@ -163,15 +161,33 @@ __global__ __launch_bounds__(kNT, 1) void bwd_dkdv_mfma(SdpaBwdParams p) {
   constexpr int LS = 2 * kTile * 4;            // their bytes per stage (lse | delta)
   __shared__ __attribute__((aligned(16))) char smem[LB + kKvStages * LS];
 #if defined(MFX_PHASE_TIMERS)
-  __shared__ unsigned ph_lds[4 * kBwdPhaseSlots * 64];
+  // Stamps of the mask-free instances only (beside a mask's registers they
+  // would spill).
+  constexpr bool TIMED = !MASK;
+  __shared__ unsigned ph_lds[TIMED ? 4 * kBwdPhaseSlots * 64 : 1];
   const int ph_lane = threadIdx.x & 63, ph_wave = threadIdx.x >> 6;
   auto ph_slot = [&](int f) -> unsigned& { return ph_lds[(ph_wave * kBwdPhaseSlots + f) * 64 + ph_lane]; };
-  auto ph_add = [&](int f, unsigned v) {
-    __hip_atomic_fetch_add(&ph_slot(f), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  auto ph_set = [&](int f, unsigned v) {
+    if constexpr (TIMED) ph_slot(f) = v;
   };
-  for (int f = 0; f < kBwdPhaseSlots; ++f) ph_slot(f) = 0;
-  ph_slot(kPhRtStart) = ph_real();
-  ph_slot(kPhCStart) = ph_now();
+  auto ph_add = [&](int f, unsigned v) {
+    if constexpr (TIMED)
+      __hip_atomic_fetch_add(&ph_slot(f), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+  auto ph_now = [&] {
+    if constexpr (TIMED) return (unsigned)__builtin_amdgcn_s_memtime();
+    else return 0u;
+  };
+  auto ph_real = [&] {
+    if constexpr (TIMED) return (unsigned)__builtin_amdgcn_s_memrealtime();
+    else return 0u;
+  };
+  auto ph_fence = [&] {
+    if constexpr (TIMED) fence();
+  };
+  for (int f = 0; f < kBwdPhaseSlots; ++f) ph_set(f, 0);
+  ph_set(kPhRtStart, ph_real());
+  ph_set(kPhCStart, ph_now());
 #endif
 
   const int tid = threadIdx.x;
@@ -437,31 +453,31 @@ __global__ __launch_bounds__(kNT, 1) void bwd_dkdv_mfma(SdpaBwdParams p) {
   auto step = [&](int t, auto ps_tag, auto pm_tag, auto st_tag, auto mt_tag) __attribute__((always_inline)) {
     constexpr int MT = decltype(mt_tag)::value;
     const int q0b = tile_q(t) * kTile + MT * 32;
-    PHASE(fence(); const unsigned c0 = ph_now(); fence();)
+    PHASE(ph_fence(); const unsigned c0 = ph_now(); ph_fence();)
     X(st_tag, mt_tag);
-    PHASE(fence(); const unsigned c1 = ph_now(); fence();)
+    PHASE(ph_fence(); const unsigned c1 = ph_now(); ph_fence();)
     const bool edge = (q0b + 32 > Tq) || (CAUSAL && q0b < kw + 31);
     if (edge)
       YV(ps_tag, pm_tag, st_tag, mt_tag, std::true_type{}, std::true_type{}, q0b);
     else
       YV(ps_tag, pm_tag, st_tag, mt_tag, std::false_type{}, std::true_type{}, q0b);
     if (MASK && (MT == 0 || t + 1 < ntiles)) mask_load(t + MT, std::integral_constant<int, 1 - MT>{});
-    PHASE(fence(); const unsigned c2 = ph_now(); ph_add(kPhX, c1 - c0); ph_add(kPhYV, c2 - c1);
-          ph_add(kPhBlocks, 1u); ph_add(kPhEdges, edge ? 1u : 0u); fence();)
+    PHASE(ph_fence(); const unsigned c2 = ph_now(); ph_add(kPhX, c1 - c0); ph_add(kPhYV, c2 - c1);
+          ph_add(kPhBlocks, 1u); ph_add(kPhEdges, edge ? 1u : 0u); ph_fence();)
   };
   // Tile t in stage ST, the previous tile in stage PS.
   auto tile = [&](int t, auto st_tag, auto ps_tag) __attribute__((always_inline)) {
     constexpr int ST = decltype(st_tag)::value;
-    PHASE(fence(); const unsigned c0 = ph_now(); fence();)
+    PHASE(ph_fence(); const unsigned c0 = ph_now(); ph_fence();)
     wait_dma();
-    PHASE(fence(); const unsigned cw = ph_now(); fence();)
+    PHASE(ph_fence(); const unsigned cw = ph_now(); ph_fence();)
     __syncthreads();
-    PHASE(fence(); const unsigned cb = ph_now(); fence();)
+    PHASE(ph_fence(); const unsigned cb = ph_now(); ph_fence();)
     // Stage (ST+1) % 3 last held tile t-2, whose last block's Y ran during
     // tile t-1, before this barrier.
     if (t + 1 < ntiles) issue(t + 1, (ST + 1) % kKvStages);
-    PHASE(fence(); const unsigned ci = ph_now(); ph_add(kPhSync, ci - c0); ph_add(kPhVmwait, cw - c0);
-          ph_add(kPhBarrier, cb - cw); ph_add(kPhTiles, 1u); fence();)
+    PHASE(ph_fence(); const unsigned ci = ph_now(); ph_add(kPhSync, ci - c0); ph_add(kPhVmwait, cw - c0);
+          ph_add(kPhBarrier, cb - cw); ph_add(kPhTiles, 1u); ph_fence();)
     step(t, ps_tag, std::integral_constant<int, 1>{}, st_tag, std::integral_constant<int, 0>{});
     step(t, st_tag, std::integral_constant<int, 0>{}, st_tag, std::integral_constant<int, 1>{});
   };
@@ -469,7 +485,7 @@ __global__ __launch_bounds__(kNT, 1) void bwd_dkdv_mfma(SdpaBwdParams p) {
   using I1 = std::integral_constant<int, 1>;
   using I2 = std::integral_constant<int, 2>;
 
-  PHASE(fence(); ph_slot(kPhRtLoop) = ph_real(); ph_slot(kPhCLoop) = ph_now(); fence();)
+  PHASE(ph_fence(); ph_set(kPhRtLoop, ph_real()); ph_set(kPhCLoop, ph_now()); ph_fence();)
   if (ntiles > 0) {
     // The first block's Y is a no-op: zero P / dS against tile 0's rows.
 #pragma unroll
@@ -487,7 +503,7 @@ __global__ __launch_bounds__(kNT, 1) void bwd_dkdv_mfma(SdpaBwdParams p) {
       tile(t + 2, I0{}, I2{});
     }
     // The last block's Y.
-    PHASE(fence(); const unsigned cl = ph_now(); fence();)
+    PHASE(ph_fence(); const unsigned cl = ph_now(); ph_fence();)
     const int ls = (ntiles - 1) % kKvStages;
     if (ls == 0)
       YV(I0{}, I1{}, I0{}, I0{}, std::false_type{}, std::false_type{}, 0);
@@ -495,10 +511,10 @@ __global__ __launch_bounds__(kNT, 1) void bwd_dkdv_mfma(SdpaBwdParams p) {
       YV(I1{}, I1{}, I0{}, I0{}, std::false_type{}, std::false_type{}, 0);
     else
       YV(I2{}, I1{}, I0{}, I0{}, std::false_type{}, std::false_type{}, 0);
-    PHASE(fence(); ph_add(kPhLast, ph_now() - cl); fence();)
+    PHASE(ph_fence(); ph_add(kPhLast, ph_now() - cl); ph_fence();)
   }
 
-  PHASE(fence(); ph_slot(kPhCEpi) = ph_now(); fence();)
+  PHASE(ph_fence(); ph_set(kPhCEpi, ph_now()); ph_fence();)
   // Every wavefront's last Y has read its Q / dO stage: the stages take the
   // dK and dV rows on their way out.  (The first key comes from an opaque
   // copy here, so no address is hoisted into the loop.)
@@ -515,7 +531,7 @@ __global__ __launch_bounds__(kNT, 1) void bwd_dkdv_mfma(SdpaBwdParams p) {
                          p.dvs[2], nvalid, dv, l32, half, lane, 1.f);
   }
 #if defined(MFX_PHASE_TIMERS)
-  {
+  if constexpr (TIMED) {
     // Fields: 0 ids (XCC id, HW_ID, (batch*Hkv + kv head), key block), 1 / 2
     // realtime start / loop entry (low words), 3 realtime end (64 bits), 4-9
     // cycles of the X phases / Y | V phases / barrier phases (all) / their
