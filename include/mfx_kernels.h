@@ -158,13 +158,19 @@ size_t mfx_layer_norm_bwd_workspace_size(const mfx_norm_bwd_args* args);
  * stays finite: a row whose keys all carry such a value returns the mean of
  * V, as jnp.where(mask, s, finite) then softmax does.
  *
+ * K and V rows that a query does not see (by causality or by -inf) take part
+ * with probability 0, or not at all where a whole tile of them is hidden: a
+ * NaN or an infinity in such a V row, and in such a K row under -inf, may or
+ * may not make the query's output NaN.  Causally hidden K rows never do.
+ *
  * q_rms_eps >= 0 applies RMSNorm over D to each query row first (rounded to
  * `dtype`, optionally times q_rms_weight[D] of `dtype`), which fuses the
  * RMSNorm(q) -> SDPA chain of GQA decode.  Pass a negative value to disable.
  *
  * dtype is MFX_F32, MFX_BF16 or MFX_F16 (fp32 accumulation for all; the
  * 16-bit paths feed probabilities rounded to `dtype` to the PV product, as
- * JAX's attention casts them to the value dtype).  Head sizes D == Dv of 32,
+ * JAX's attention casts them to the value dtype; unrounded at head sizes 32
+ * and 96 with a mask that varies along queries, and on the per-row kernel).  Head sizes D == Dv of 32,
  * 64, 96, 128 and 256 run on the matrix-core kernels (mfx_sdpa_kernel_name
  * names the one a call takes); any other up to 256 on a per-row kernel.
  *
@@ -259,7 +265,10 @@ const char* mfx_sdpa_kernel_name(const mfx_sdpa_args* args);
  * custom_call @mlx_sdpa_bwd interface (q, k, v, grad_out) has no slot for
  * them, and its mx::vjp recomputes.  Workspace:
  * mfx_sdpa_bwd_workspace_size() bytes, or NULL for library scratch.
- * Deterministic: no atomics.  dq, dk and dv must not share memory with the
+ * Deterministic: no atomics.  NaN and infinities in rows that causality hides
+ * reach no gradient in f32 calls (from forward results that are finite
+ * themselves); the 16-bit matrix-core kernels multiply such rows by zero, and
+ * rows under -inf may count or not, as in the forward.  dq, dk and dv must not share memory with the
  * inputs or each other; only f32 calls may store dq over q or dout, row by row
  * (on the per-row kernels, a slower route).
  * Replaces mx::vjp of fast::scaled_dot_product_attention behind custom_call

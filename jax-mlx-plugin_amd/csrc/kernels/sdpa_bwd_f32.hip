@@ -25,9 +25,15 @@
 //
 // Measured on [32,256,8,64] BTNH without a mask: dQ 69 us (93 TFLOP/s) and
 // dK / dV 89 us (97), against 1177 and 7445 us for the one-wavefront-per-row
-// kernels (sdpa_bwd.hip) that ran these calls before; the whole recomputing
-// call 193 against 8653 us, and [1,1,32,64] 24 against 38, so every call that
-// meets bwd_f32_supports comes here.
+// kernels (sdpa_bwd.hip) that ran these calls before, the matrix cores 60-63%
+// busy; the whole recomputing call 181 against 8712 us.  Every call that meets
+// bwd_f32_supports comes here: also where a wavefront walks all its tiles alone
+// the per-row kernels, whose wavefronts walk as many rows one by one, take
+// longer (from residuals at D = 64, this file against theirs in us: one tile
+// [1,1,32] 14 and 30; 8 heads over 1 kv head, 4096 queries, 64 keys 4957 and
+// 14767; 64 over 1, 512 queries, one key 4939 and 14648; one query, 8192 keys
+// 914 and 1575; 64 heads of one query and one key 14 and 17; at D = 32 to 128
+// over 96 such shapes 0.03 to 0.87 of their time).
 #include "sdpa_f32.h"
 
 namespace mfx {

@@ -297,10 +297,11 @@ __global__ __launch_bounds__(kNT, 1) void bwd_dkdv_mfma(SdpaBwdParams p) {
   }
   const uint32_t la = base + LB + half * 16;  // lse | delta of rows 4*half ..
 
-  // The mask values of a block's 16 rows at this lane's key, all in flight
-  // from the end of the block before.  Loaded where they were used, each
-  // behind a branch on the type, they took more time than the products
-  // (sdpa_mask.h).
+  // The mask values of a block's 16 rows at this lane's key, loaded together at
+  // the end of the block before: a tile's second block finds them there, its
+  // first waits for them with the tile's own loads (wait_dma).  Loaded where
+  // they were used, each behind a branch on the type, they took more time than
+  // the products (sdpa_mask.h).
   // (As loaded: 16-bit types convert at their use.)
   uint32_t mv[MASK ? 16 : 1];
   using MElem = std::conditional_t<MASKT == 2 || MASKT == 3, uint16_t, uint32_t>;

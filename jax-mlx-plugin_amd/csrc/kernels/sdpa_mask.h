@@ -5,9 +5,11 @@
 // Loading whole runs is what makes this kernel fast: one element at a time
 // behind a branch on the type, each load waited for alone, a
 // [1,16,1999,1999] bf16 bias took 1045 us a call on [4,16,1999,128] GQA;
-// in runs, a tile's all in flight a tile ahead, 221 (179 with 2048 keys,
-// against 129 without a mask: what is left is the mask's own vector work
-// and its loads, 32 rows of 32 bytes each).  The backward of the same call
+// in runs, a tile's all in flight a tile ahead, 214 (187 with 2048 keys, whose
+// rows start on a dword; 132 to 145 without a mask on the pipelined kernel).
+// What is left is the mask's own vector work, 12 vector instructions a matrix
+// instruction where there are 4.6 without a mask: the vector units are busy
+// 51-56% of the time and the matrix cores 29-34%.  The backward of the same call
 // from its residuals went from 2511 to 812 us (padding mask: 1444 to 754).
 #pragma once
 
