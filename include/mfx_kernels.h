@@ -134,7 +134,8 @@ typedef struct {
 
 int mfx_layer_norm_bwd(const mfx_norm_bwd_args* args, void* stream);
 
-/* Bytes of workspace mfx_layer_norm_bwd needs for these arguments. */
+/* Bytes of workspace mfx_layer_norm_bwd needs for these arguments, at any
+ * alignment of the tensors. */
 size_t mfx_layer_norm_bwd_workspace_size(const mfx_norm_bwd_args* args);
 
 /*

@@ -18,6 +18,8 @@
 // (workspace [G][2][n]).  Pass 2 (ln_bwd_params) sums the G partials per
 // column.  HBM traffic: x and dy read once, dx written once, plus
 // 2 * G * n * 4 bytes of partials written and read back.
+#include <algorithm>
+
 #include "rowvec.h"
 
 namespace mfx {
@@ -452,7 +454,8 @@ struct BwdPlan {
 
 int vec_of(int dt) { return dt == MFX_F32 ? 4 : 8; }
 
-BwdPlan plan_bwd(const mfx_norm_bwd_args& a) {
+// off16: as for tensors off 16 bytes, whatever the pointers are.
+BwdPlan plan_bwd(const mfx_norm_bwd_args& a, bool off16 = false) {
   BwdPlan p;
   const int VEC = vec_of(a.dtype);
   const int pbytes = a.param_dtype == MFX_F32 ? 4 : 2;
@@ -461,7 +464,7 @@ BwdPlan plan_bwd(const mfx_norm_bwd_args& a) {
   // bf16 (f16 rows: f32 or f16).
   const bool ptype = !a.gamma || a.param_dtype == MFX_F32 ||
                      a.param_dtype == (a.dtype == MFX_F16 ? MFX_F16 : MFX_BF16);
-  const bool aligned = a.n % VEC == 0 && a.x_row_stride % VEC == 0 && a.dy_row_stride % VEC == 0 &&
+  const bool aligned = !off16 && a.n % VEC == 0 && a.x_row_stride % VEC == 0 && a.dy_row_stride % VEC == 0 &&
                        a.dx_row_stride % VEC == 0 && (uintptr_t)a.x % 16 == 0 &&
                        (uintptr_t)a.dy % 16 == 0 && (uintptr_t)a.dx % 16 == 0 &&
                        (!a.gamma || (uintptr_t)a.gamma % palign == 0);
@@ -573,7 +576,7 @@ extern "C" {
 size_t mfx_layer_norm_bwd_workspace_size(const mfx_norm_bwd_args* args) {
   using namespace mfx;
   if (validate(args)) return 0;
-  return partial_bytes(*args, plan_bwd(*args));
+  return std::max(partial_bytes(*args, plan_bwd(*args)), partial_bytes(*args, plan_bwd(*args, true)));
 }
 
 int mfx_layer_norm_bwd(const mfx_norm_bwd_args* args, void* stream) {

@@ -227,6 +227,19 @@ def test_layer_norm_bwd_rows_of_any_length_and_alignment(cuda, nat, oracle, dt, 
                 assert np.abs(o - r).max() <= (BF16_REL_TOL if dt == "bf16" else F16_REL_TOL) * max(np.abs(r).max(), 1e-3)
 
 
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("rows,n", [(1, 64), (8, 256), (100, 256), (128, 64), (200, 256), (100, 512), (65, 4096), (70, 8192)])
+def test_layer_norm_bwd_workspace_of_unaligned_views(cuda, nat, dt, rows, n):
+    """A workspace of the queried size serves views off 16 bytes, with the
+    same bits as the library's own."""
+    td = {"f32": cuda.float32, "bf16": cuda.bfloat16}[dt]
+    x = cuda.randn(rows * n + 1, device="cuda").to(td)[1:].view(rows, n)
+    dy = cuda.randn(rows, n, device="cuda").to(td)
+    ws = cuda.empty(nat.layer_norm_bwd_workspace_size(x), dtype=cuda.uint8, device="cuda")
+    for a, b in zip(nat.layer_norm_bwd(x, dy, workspace=ws), nat.layer_norm_bwd(x, dy)):
+        assert cuda.equal(a, b)
+
+
 @pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
 @pytest.mark.parametrize("n", [64, 511, 512, 4096, 4097])
 @pytest.mark.parametrize("rows", [1, 3, 2049])
