@@ -154,14 +154,37 @@ __device__ __forceinline__ void store_row(float* row, const f32x16 (&acc)[D / 32
     }
 }
 
+// Bit r: row r of 32 (n of them there) holds a NaN or an infinity; with ALL,
+// nothing but NaN.
+template <int D, bool ALL>
+__device__ __forceinline__ uint32_t odd_rows(const float* rows, int64_t stride, int n, int l32, int half) {
+  if (n <= 0) return 0;
+  const float* row = rows + min(l32, n - 1) * stride + half * 4;
+  bool any = false, all = true;
+#pragma unroll 2
+  for (int c = 0; c < D / 8; ++c) {
+    const f32x4 a = *reinterpret_cast<const f32x4*>(row + c * 8);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float z = a[e] * 0.f;  // NaN unless finite
+      any |= z != z;
+      all &= a[e] != a[e];
+    }
+  }
+  const uint64_t b = __ballot(l32 < n && (ALL ? all : any));
+  return ALL ? (uint32_t)b & (uint32_t)(b >> 32) : (uint32_t)b | (uint32_t)(b >> 32);
+}
+
 // A matrix product multiplies the rows that causality hides too, by zero,
 // which is NaN where such a row is not finite; but hidden rows must not take
-// part at all.  So where a causal call's sums are not all finite, the
-// wavefront's 32 output rows are computed again by these, one row at a time
-// from what it sees: a lane per row of the other axis for the scores, then per
-// feature for the sums.  (Asking the sums costs D / 2 instructions, D in dkdv,
-// once a wavefront: [16,8,20,64] goes from 14.9 to 15.3 us, [1,1,2048,64] stays
-// at 539.)
+// part at all.  They lie in the tile on a wavefront's diagonal.  So where a
+// causal call's sums are not all finite, the rows among the wavefront's 32 that
+// hide such a row, and are not NaN throughout by what they see, are computed
+// again by these, one at a time from what the row sees: a lane per row of the
+// other axis for the scores, then per feature for the sums.  (Asking the sums
+// costs D / 2 instructions, D in dkdv, once a wavefront: [16,8,20,64] goes from
+// 14.9 to 15.2 us, [1,1,2048,64] stays at 538, and K of NaN throughout costs
+// [1,8,2048,64] GQA 2% of its 2.85 ms.)
 //
 // Features f*64 + lane of a row.
 template <int D>
@@ -340,13 +363,19 @@ __global__ __launch_bounds__(64 * NW, D <= 64 ? 2 : 1) void bwd_f32_dq_kernel(Sd
     if (t + 1 < ntiles) ld.store(k_lds[(t + 1) & 1], v_lds[(t + 1) & 1], tid);
     __syncthreads();
   }
+  uint32_t again = 0;  // rows for dq_row
   if (causal && __builtin_expect(nonfinite<D>(dq), false)) {
-    for (int r = 0; r < 32 && q0 + r < Tq; ++r)
-      dq_row<D, MT>(p, b, h, q0 + r, __shfl(lse, r, 64), __shfl(delta, r, 64), lane);
-    return;
+    const uint32_t odd = odd_rows<D, false>(kp + (int64_t)q0 * ks2, ks2, min(32, Tk - q0), l32, half);
+    // A NaN lse or delta makes the whole row NaN.
+    const bool nan = lse != lse || delta != delta;
+    again = (uint32_t)__ballot(qv && !nan && (odd >> l32 >> 1) != 0);
   }
-  if (qv)
+  if (qv && !(again >> l32 & 1))
     store_row<D>(static_cast<float*>(p.dq) + b * p.dqs[0] + h * p.dqs[1] + (int64_t)qi * p.dqs[2], dq, half, p.scale);
+  for (; again; again &= again - 1) {
+    const int r = __builtin_ctz(again);
+    dq_row<D, MT>(p, b, h, q0 + r, __shfl(lse, r, 64), __shfl(delta, r, 64), lane);
+  }
 }
 
 template <int D, int NW, int MT>
@@ -439,14 +468,37 @@ __global__ __launch_bounds__(64 * NW, D <= 64 ? 2 : 1) void bwd_f32_dkdv_kernel(
     if (it + 1 < n) store((it + 1) & 1);
     __syncthreads();
   }
+  uint32_t again = 0;  // rows for dkdv_row
   if (causal && __builtin_expect(nonfinite<D>(dk) || nonfinite<D>(dv), false)) {
-    for (int r = 0; r < 32 && k0 + r < Tk; ++r) dkdv_row<D, MT>(p, b, hk, k0 + r, lane);
-    return;
+    uint32_t odd = 0, blank = 0;       // of the diagonal's query rows, in any head: not finite, dO all NaN
+    int nan_lse = -1, nan_delta = -1;  // the last such query
+    for (int h = hk * G; h < (hk + 1) * G; ++h) {
+      const float* q = static_cast<const float*>(p.q) + b * p.qs[0] + h * p.qs[1] + (int64_t)k0 * qs2;
+      const float* g = static_cast<const float*>(p.dout) + b * p.dos[0] + h * p.dos[1] + (int64_t)k0 * gs2;
+      const int m = min(32, Tq - k0);
+      odd |= odd_rows<D, false>(q, qs2, m, l32, half) | odd_rows<D, false>(g, gs2, m, l32, half);
+      blank |= odd_rows<D, true>(g, gs2, m, l32, half);
+      const int64_t rows = ((int64_t)b * p.Hq + h) * Tq;
+      for (int i = k0 + lane; i < Tq; i += 64) {
+        if (p.lse[rows + i] != p.lse[rows + i]) nan_lse = max(nan_lse, i);
+        if (p.delta[rows + i] != p.delta[rows + i]) nan_delta = max(nan_delta, i);
+      }
+    }
+#pragma unroll
+    for (int o = 32; o; o >>= 1) {
+      nan_lse = max(nan_lse, __shfl_xor(nan_lse, o, 64));
+      nan_delta = max(nan_delta, __shfl_xor(nan_delta, o, 64));
+    }
+    // A query with a NaN lse makes dK and dV of all it sees NaN, a NaN delta
+    // dK; the key's own query dV where its dO is.
+    const bool nan = key <= nan_lse || (key <= nan_delta && (blank >> l32 & 1));
+    again = (uint32_t)__ballot(key < Tk && !nan && (odd & ((1u << l32) - 1)) != 0);
   }
-  if (key < Tk) {
+  if (key < Tk && !(again >> l32 & 1)) {
     store_row<D>(static_cast<float*>(p.dk) + b * p.dks[0] + hk * p.dks[1] + (int64_t)key * p.dks[2], dk, half, p.scale);
     store_row<D>(static_cast<float*>(p.dv) + b * p.dvs[0] + hk * p.dvs[1] + (int64_t)key * p.dvs[2], dv, half, 1.f);
   }
+  for (; again; again &= again - 1) dkdv_row<D, MT>(p, b, hk, k0 + __builtin_ctz(again), lane);
 }
 
 // Wavefronts per workgroup of a kernel whose wavefronts own 32 of T rows in
